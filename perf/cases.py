@@ -237,7 +237,7 @@ def prepare(case, seed):
     if kind == "batch":
         sims, r = [], np.random.default_rng(seed)
         for k, (system, stepper, observer) in enumerate((("van_der_pol", "dopri5", "thresh2"),
-                                                         ("lorenz", "dopri5", "basicall"),
+                                                         ("lactotroph", "rk4", "basicall"),
                                                          ("chay_keizer", "dopri5", "localmax"),
                                                          ("ornstein_uhlenbeck", "seuler", "basicall"))):
             sim = clode.FeatureSimulator(observer=OBSERVERS[observer], observer_x_up_thresh=0.3,
@@ -327,7 +327,7 @@ def work(case):
     if kind == "batch":
         n, span = case["members"], 1.65 * case["span"]  # the mean of exp(z), z ~ N(0, 1)
         flops = sum(p * n * _steps(case, s, st, span) * _step_flops(s, st) for s, st, p in
-                    (("van_der_pol", "dopri5", 3), ("lorenz", "dopri5", 2), ("chay_keizer", "dopri5", 2),
+                    (("van_der_pol", "dopri5", 3), ("lactotroph", "rk4", 2), ("chay_keizer", "dopri5", 2),
                      ("ornstein_uhlenbeck", "seuler", 2)))
         return {"bytes": n * 1500, "flops": flops}
     if kind == "train":
