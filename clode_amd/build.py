@@ -31,6 +31,7 @@ ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 DEVICE_HEADERS = [
     "cm_math.h",
     "clode_builtins.h",
+    "clode_divide.h",
     "clode_prelude.h",
     "clode_layout.h",
     "clode_kernel_args.h",

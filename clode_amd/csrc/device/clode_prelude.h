@@ -74,5 +74,11 @@ typedef double timetype;
 
 #include "cm_math.h"
 #include "clode_builtins.h"
+#if CLODE_PREC != 3
+#include "clode_divide.h"
+#define CLODE_DIVIDE(x, y) clode_div::divide<realtype>(x, y)
+#else
+#define CLODE_DIVIDE(x, y) ((x) / (y))
+#endif
 
 #endif  // CLODE_PRELUDE_H

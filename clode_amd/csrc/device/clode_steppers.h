@@ -147,7 +147,7 @@ CLODE_DEV void do_step(realtype &ti, realtype xi[], realtype k1[], const realtyp
         tmp[k] = xi[k] + dt * k3[k];
     getRHS(th, tmp, pars, k4, aux, wi);
     for (int k = 0; k < N_VAR; k++)
-        xi[k] += dt * (k1[k] + RCONST(2.0) * k2[k] + RCONST(2.0) * k3[k] + k4[k]) / RCONST(6.0);
+        xi[k] += CLODE_DIVIDE(dt * (k1[k] + RCONST(2.0) * k2[k] + RCONST(2.0) * k3[k] + k4[k]), RCONST(6.0));
     ti = th;
 }
 #endif

@@ -68,8 +68,7 @@ void Batch::compileOnly(const std::vector<Simulator *> &sims)
             throw InvalidArgument("null simulator in batch");
         cfgs.push_back(s->programConfig());
     }
-    std::string src = compose_batch_source(cfgs);
-    get_program_source(src, compile_options(cfgs[0]), sims[0]->root);
+    get_batch_program(cfgs, sims[0]->root);
 }
 
 std::shared_ptr<Program> Batch::program()
@@ -79,7 +78,7 @@ std::shared_ptr<Program> Batch::program()
         cfgs.push_back(s->programConfig());
     std::string src = compose_batch_source(cfgs);
     if (!prog_ || src != progKey_) {
-        prog_ = get_program_source(src, compile_options(cfgs[0]), sims_[0]->root);
+        prog_ = get_batch_program(cfgs, sims_[0]->root);
         progKey_ = src;
     }
     return prog_;

@@ -90,6 +90,7 @@ struct ProgramConfig {
     int nVar = 0, nPar = 0, nAux = 0, nWiener = 0, nStore = 0;
     int wavesPerEU = 0;  // > 0: kernels compiled for at least this many waves per SIMD
     bool replay = false;  // also the warm-up record / features replay kernels
+    bool plainDivision = false;  // the right-hand side's divisions as written (see division_operators)
     std::string rhs;
     std::string rhs_name;
 };
@@ -107,16 +108,20 @@ private:
     std::map<int, hipModule_t> modules_;
 };
 
+// a right-hand side with its "/" tokens inside function bodies replaced by the
+// named operator of clode_divide.h
+std::string division_operators(const std::string &rhs);
 std::string compose_source(const ProgramConfig &cfg);
 // toolchain text mixed into every program's cache key
 std::string toolchain_identity();
 std::vector<std::string> compile_options(const ProgramConfig &cfg);
 std::shared_ptr<Program> get_program(const ProgramConfig &cfg, const std::string &cache_dir);
 std::shared_ptr<Program> get_program_source(const std::string &source, const std::vector<std::string> &options,
-                                            const std::string &cache_dir);
+                                            const std::string &cache_dir, bool report = true);
 
 // batched programs: up to CLODE_BATCH_MAX systems in one code object
 constexpr size_t CLODE_BATCH_MAX = 8;
 std::string compose_batch_source(const std::vector<ProgramConfig> &cfgs);
+std::shared_ptr<Program> get_batch_program(std::vector<ProgramConfig> cfgs, const std::string &cache_dir);
 
 }  // namespace clode

@@ -10,6 +10,7 @@
 
 #include <hip/hiprtc.h>
 
+#include <cctype>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
@@ -224,6 +225,80 @@ void DeviceBuffer::release()
 }
 
 // ------------------------------------------------------------------ program
+
+// The token "/" becomes " *CLODE_DIV* ", which has the same precedence and
+// associativity, so every expression keeps its tree.  Left alone: comments,
+// character and string literals, preprocessor lines (macro bodies keep their
+// divisions), "/=", and everything outside braces.
+std::string division_operators(const std::string &rhs)
+{
+    std::string out;
+    out.reserve(rhs.size() + 256);
+    const size_t n = rhs.size();
+    int depth = 0;
+    bool lineStart = true;  // only blanks since the last line break
+    auto spliced = [&](size_t i) {  // the line break at i follows a backslash
+        return (i > 0 && rhs[i - 1] == '\\') || (i > 1 && rhs[i - 1] == '\r' && rhs[i - 2] == '\\');
+    };
+    // up to (not including) the end of the logical line
+    auto copyLine = [&](size_t i) {
+        while (i < n && (rhs[i] != '\n' || spliced(i)))
+            out += rhs[i++];
+        return i;
+    };
+    for (size_t i = 0; i < n;) {
+        const char c = rhs[i], d = i + 1 < n ? rhs[i + 1] : '\0';
+        if (c == '#' && lineStart) {
+            i = copyLine(i);
+            continue;
+        }
+        if (c == '/' && d == '/') {
+            i = copyLine(i);
+            continue;
+        }
+        if (c == '/' && d == '*') {
+            const size_t e = rhs.find("*/", i + 2), stop = e == std::string::npos ? n : e + 2;
+            out.append(rhs, i, stop - i);
+            i = stop;
+            continue;
+        }
+        // a quote starts a literal, except as a digit separator (1'000)
+        if (c == '"' || (c == '\'' && !(i > 0 && (std::isalnum((unsigned char)rhs[i - 1]) || rhs[i - 1] == '_')))) {
+            out += c;
+            for (++i; i < n && rhs[i] != c && rhs[i] != '\n'; ++i) {
+                out += rhs[i];
+                if (rhs[i] == '\\' && i + 1 < n)
+                    out += rhs[++i];
+            }
+            if (i < n)
+                out += rhs[i++];
+            lineStart = false;
+            continue;
+        }
+        if (c == '{')
+            ++depth;
+        else if (c == '}')
+            --depth;
+        if (c == '/' && depth > 0 && d != '=')
+            out += " *CLODE_DIV* ";
+        else
+            out += c;
+        if (c == '\n')
+            lineStart = true;
+        else if (c != ' ' && c != '\t' && c != '\r')
+            lineStart = false;
+        ++i;
+    }
+    return out;
+}
+
+// The right-hand side as compiled.  fp32c programs divide by reciprocals
+// (compile_options) and keep the text.
+static std::string program_rhs(const ProgramConfig &cfg)
+{
+    return cfg.prec == PREC_FP32C || cfg.plainDivision ? cfg.rhs : division_operators(cfg.rhs);
+}
+
 std::string compose_source(const ProgramConfig &cfg)
 {
     std::ostringstream s;
@@ -253,7 +328,7 @@ std::string compose_source(const ProgramConfig &cfg)
     if (slash != std::string::npos)
         rname = rname.substr(slash + 1);
     s << "#line 1 \"" << rname << "\"\n";
-    s << cfg.rhs << "\n";
+    s << program_rhs(cfg) << "\n";
     s << "#pragma clang force_cuda_host_device end\n";
     s << "#include \"clode_rng.h\"\n";
     s << "#include \"clode_steppers.h\"\n";
@@ -286,7 +361,7 @@ static void compose_system(std::ostringstream &s, const ProgramConfig &cfg, size
     if (slash != std::string::npos)
         rname = rname.substr(slash + 1);
     s << "#line 1 \"" << rname << "\"\n";
-    s << cfg.rhs << "\n";
+    s << program_rhs(cfg) << "\n";
     s << "#pragma clang force_cuda_host_device end\n";
     s << "#include \"clode_steppers.h\"\n";
     if (cfg.observer > 0)
@@ -524,13 +599,42 @@ static void rtc_check(hiprtcResult r, const char *what)
         throw RuntimeError(std::string(what) + ": " + hiprtcGetErrorString(r));
 }
 
+// A right-hand side that the compiler refuses with its divisions replaced is
+// compiled as written; errors are then those of the user's own text.
 std::shared_ptr<Program> get_program(const ProgramConfig &cfg, const std::string &cache_dir)
 {
-    return get_program_source(compose_source(cfg), compile_options(cfg), cache_dir);
+    ProgramConfig plain = cfg;
+    plain.plainDivision = true;
+    const std::string source = compose_source(cfg), asWritten = compose_source(plain);
+    if (source != asWritten) {
+        try {
+            return get_program_source(source, compile_options(cfg), cache_dir, false);
+        } catch (const RuntimeError &) {
+            log_msg(LOG_DEBUG, "right-hand side compiled with its divisions as written");
+        }
+    }
+    return get_program_source(asWritten, compile_options(plain), cache_dir);
+}
+
+std::shared_ptr<Program> get_batch_program(std::vector<ProgramConfig> cfgs, const std::string &cache_dir)
+{
+    const std::string source = compose_batch_source(cfgs);
+    const std::vector<std::string> options = compile_options(cfgs[0]);
+    for (auto &c : cfgs)
+        c.plainDivision = true;
+    const std::string asWritten = compose_batch_source(cfgs);
+    if (source != asWritten) {
+        try {
+            return get_program_source(source, options, cache_dir, false);
+        } catch (const RuntimeError &) {
+            log_msg(LOG_DEBUG, "right-hand sides compiled with their divisions as written");
+        }
+    }
+    return get_program_source(asWritten, options, cache_dir);
 }
 
 std::shared_ptr<Program> get_program_source(const std::string &source, const std::vector<std::string> &options,
-                                            const std::string &cache_dir)
+                                            const std::string &cache_dir, bool report)
 {
     auto prog = std::make_shared<Program>();
     prog->source = source;
@@ -546,8 +650,10 @@ std::shared_ptr<Program> get_program_source(const std::string &source, const std
 
     std::lock_guard<std::mutex> lk(g_prog_mu);
     auto it = g_programs.find(key);
-    if (it != g_programs.end())
+    if (it != g_programs.end() && it->second)
         return it->second;
+    if (it != g_programs.end() && !report)  // known to fail
+        throw RuntimeError("hipRTC build failed");
 
     const std::string path = cache_dir.empty() ? std::string() : cache_path(cache_dir, key);
     if (!path.empty() && read_cache(path, key, prog->code)) {
@@ -573,7 +679,9 @@ std::shared_ptr<Program> get_program_source(const std::string &source, const std
             hiprtcGetProgramLog(p, &buildlog[0]);
         if (r != HIPRTC_SUCCESS) {
             hiprtcDestroyProgram(&p);
-            log_msg(LOG_ERR, "hipRTC build failed:\n" + buildlog);
+            if (!report)
+                g_programs[key] = nullptr;
+            log_msg(report ? LOG_ERR : LOG_DEBUG, "hipRTC build failed:\n" + buildlog);
             throw RuntimeError("hipRTC build failed: " + buildlog);
         }
         if (logsize > 1)

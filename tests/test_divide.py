@@ -1,0 +1,125 @@
+"""Divisions of a right-hand side (clode_divide.h): which tokens the program builder replaces, that what it cannot
+replace still compiles, and that the quotients by constants are those of IEEE division."""
+import os
+
+import numpy as np
+import pytest
+
+import clode_amd as clode
+from clode_amd.cpp import clode_cpp_wrapper as w
+
+HEAD = ("void getRHS(const realtype t, const realtype x_[], const realtype p_[], realtype dx_[], realtype aux_[], "
+        "const realtype w_[])\n{\n")
+
+
+def _program(tmp_path, text, precision, compile=False):
+    path = tmp_path / "rhs.cl"
+    path.write_text(text)
+    pi = w.ProblemInfo(str(path), ["x"], ["p"], [], 0)
+    sim = w.SimulatorBase(pi, "euler", precision, w.OpenCLResource(), str(tmp_path / "cache"))
+    if compile:
+        sim.compile()
+    s = sim.get_program_string()
+    return s[s.index('#line 1 "rhs.cl"'):s.index("clode_rng.h")]
+
+
+@pytest.mark.parametrize("line, out", [
+    ("dx_[0] = a / b;", "dx_[0] = a  *CLODE_DIV*  b;"),
+    ("dx_[0] = a/b/c;", "dx_[0] = a *CLODE_DIV* b *CLODE_DIV* c;"),
+    ("a /= b;", "a /= b;"),
+    ("a = 1; // a / b", "a = 1; // a / b"),
+    ("a = b /* x / y */ / c;", "a = b /* x / y */  *CLODE_DIV*  c;"),
+    ("a = 1; // a \\\n / b", "a = 1; // a \\\n / b"),
+    ("#define F(x) ((x) / \\\n 3.0)\na = F(b) / 2;", "#define F(x) ((x) / \\\n 3.0)\na = F(b)  *CLODE_DIV*  2;"),
+    ("const char *s = \"a / \\\" / b\"; char c = '/';", "const char *s = \"a / \\\" / b\"; char c = '/';"),
+    ("a = 1'000.0 / b;", "a = 1'000.0  *CLODE_DIV*  b;"),
+])
+def test_replaced_tokens(tmp_path, line, out):
+    assert out in _program(tmp_path, HEAD + line + "\n}\n", False)
+    assert line in _program(tmp_path, HEAD + line + "\n}\n", "fp32c")  # divides by reciprocals instead
+
+
+def test_outside_functions_as_written(tmp_path):
+    text = "const int half = 7 / 2;\n" + HEAD + "dx_[0] = p_[0] / half;\n}\n"
+    s = _program(tmp_path, text, False)
+    assert "half = 7 / 2;" in s and "p_[0]  *CLODE_DIV*  half" in s
+
+
+# forms of "/" whose operands or results are not plain real numbers; the last cannot go through the operator (its
+# left side cannot be copied) and compiles as written
+FORMS = {
+    "integers": "enum { K = 6 / 2 }; int a[8 / 4]; a[1] = 7 / 2; switch (a[1]) { case 9 / 3: dx_[0] = a[1] / K; }",
+    "mixed": "float f = 3.5f; int n = 3; dx_[0] = n / f + f / n + p_[0] / n + 1 / p_[0] + 5 / n;",
+    "pointer": "const realtype *q = p_; dx_[0] = x_[0] / *q / -*q;",
+    "size": "realtype a[3]; dx_[0] = p_[0] / (sizeof(a) / sizeof(a[0]));",
+    "lambda": "auto f = [](auto a, auto b) { return a / b; }; dx_[0] = f(p_[0], 12) + f(7, 2);",
+    "constants": "const realtype c = RCONST(1.0) / RCONST(3.0); dx_[0] = c / RCONST(7.0) + 0.0 / 1.0;",
+    "vector": "double2 v = make_double2(p_[0], 1.0); dx_[0] = (v / 3.0).x;",
+    "own type": "struct R { double v; R(double a) : v(a) {} R(const R &) = delete; double operator/(double d) const "
+                "{ return v / d; } }; R r(p_[0]); dx_[0] = r / 3.0;",
+}
+
+
+@pytest.mark.parametrize("precision", [True, False])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_forms_compile(tmp_path, form, precision):
+    _program(tmp_path, HEAD + FORMS[form] + "\n}\n", precision, compile=True)
+
+
+def _quotients(tmp_path, divisor, p, precision):
+    """p / divisor as the right-hand side computes it: one Euler step of length 1 from x = 0."""
+    path = tmp_path / "q.cl"
+    path.write_text(HEAD + f"const realtype c = {divisor};\ndx_[0] = p_[0] / c;\n}}\n")
+    sim = clode.Simulator(src_file=str(path), variables={"x": 0.0}, parameters={"p": 1.0},
+                          stepper=clode.Stepper.euler, dt=1.0, t_span=(0.0, 0.5), single_precision=precision)
+    sim.set_ensemble(variables=np.zeros((p.size, 1)), parameters=p.astype(np.float64)[:, None])
+    return np.ravel(sim.transient(update_x0=False, fetch_results=True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [True, False])
+@pytest.mark.parametrize("divisor", ["3", "10", "12.0", "-30", "6", "5300", "524287", "524288.0", "524289", "1000003",
+                                     "281474976710655.0", "281474976710657.0", "0.1", "2.5", "8", "1", "-1", "0"])
+def test_quotients_by_constants(tmp_path, divisor, precision):
+    T, U = (np.float32, np.uint32) if precision else (np.float64, np.uint64)
+    r = np.random.default_rng(int(abs(float(divisor))) % 1000)
+    c = T(float(divisor))
+    tiny = np.finfo(T).tiny
+    big = np.finfo(T).max
+    anybits = r.integers(0, np.iinfo(U).max, 20000, dtype=U, endpoint=True).view(T)
+    # numerators next to c times a middle between two neighbours, where a quotient is hardest to round
+    m = (1 + r.random(20000)).astype(T)
+    with np.errstate(all="ignore"):
+        near = (m * c).astype(T)
+        near = (near.view(U) + r.integers(0, 5, near.size).astype(U) - U(2)).view(T)
+        special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, tiny, -tiny, big, -big, 1.0, c, -c, c * tiny], T)
+        p = np.concatenate([anybits, near, special])
+        want = p / c
+        got = _quotients(tmp_path, divisor, p, precision).astype(T)
+    # a subnormal quotient by an even number may be a middle itself: either neighbour is as near
+    tie = np.zeros(p.size, bool)
+    if c != 0 and float(c) % 2 == 0 and abs(float(c)) > 2:
+        tie = (np.abs(want) < tiny) & np.isfinite(want)
+        unit = np.nextafter(T(0), T(1))
+        assert np.all(np.abs(got[tie] - want[tie]) <= unit)
+    want = want + T(0)  # x = 0 + 1 * (p / c)
+    same = (got.view(U) == want.view(U)) | (np.isnan(got) & np.isnan(want))
+    assert np.all(same | tie), (p[~(same | tie)][:5], got[~(same | tie)][:5], want[~(same | tie)][:5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [True, False])
+def test_forms_values(tmp_path, precision):
+    """The mixed and integer forms give the values of C."""
+    path = tmp_path / "q.cl"
+    path.write_text(HEAD + "int n = 3; float f = 3.5f;\n"
+                    "dx_[0] = p_[0] / n + 7 / 2 + n / f + 1 / p_[0] + 7 / -n + (p_[0] - 5 / 2) / 12 / f;\n}\n")
+    T = np.float32 if precision else np.float64
+    p = np.linspace(0.5, 9.0, 100).astype(T)
+    sim = clode.Simulator(src_file=str(path), variables={"x": 0.0}, parameters={"p": 1.0},
+                          stepper=clode.Stepper.euler, dt=1.0, t_span=(0.0, 0.5), single_precision=precision)
+    sim.set_ensemble(variables=np.zeros((p.size, 1)), parameters=p.astype(np.float64)[:, None])
+    got = np.ravel(sim.transient(update_x0=False, fetch_results=True)).astype(T)
+    f = np.float32(3.5)
+    want = p / T(3) + T(3) + T(np.float32(3) / f) + T(1) / p + T(-2) + (p - T(2)) / T(12) / T(f)
+    np.testing.assert_array_equal(got, want)
