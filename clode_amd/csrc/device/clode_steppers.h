@@ -73,8 +73,10 @@ struct SolverParamsR {
 // The drivers call step_attempt() once per loop iteration.  A fixed-step
 // stepper completes its step in one attempt.  The adaptive controller makes
 // one trial per attempt and keeps what its retry loop carries between trials
-// (adaptive_explicit_step.clh:14-62: the trial step size, the attempt count
-// and whether a trial has failed) in StepCtl, so a lane whose trial was
+// (adaptive_explicit_step.clh:14-62): the trial step size in dt itself (dt is
+// read by nobody until the step is done, and the finished step overwrites
+// it), the attempt count and the previous trial's step in StepCtl.  Whether a
+// trial of this step has failed is attempts != 0.  So a lane whose trial was
 // rejected retries on the next iteration while the other lanes of its wave go
 // on with their next steps.  Each member still sees exactly the reference's
 // sequence of trials; only the interleaving across lanes changes.
@@ -84,20 +86,37 @@ typedef double ctlreal;
 typedef realtype ctlreal;
 #endif
 struct StepCtl {
-    ctlreal newDt;   // the next trial's step before clamping
     ctlreal lastDt;  // the previous trial's clamped step (stall detection)
-    int attempts;
-    bool noFailedSteps;
-    bool inStep;
+    int attempts;    // trials made of the current step: 0 at its start
 };
 CLODE_DEV void step_ctl_reset(StepCtl &c)
 {
-    c.newDt = 0;
     c.lastDt = 0;
     c.attempts = 0;
-    c.noFailedSteps = true;
-    c.inStep = false;
 }
+
+// cm::min_step for the lanes of a wave.  All but the first steps of a run from
+// t = 0 are at a positive time stepping upward, where the result is t's
+// exponent field less 48 (19 in float); one test for the whole wave then
+// replaces the formula's branches.  Any other lane sends the wave there.
+#if defined(CLODE_ADAPTIVE_STEP)
+CLODE_DEV double wave_min_step(double t, double toward)
+{
+    const unsigned int hi = (unsigned int)((unsigned long long)__double_as_longlong(t) >> 32);
+    const bool plain = hi - 0x03100000u < 0x7fe00000u - 0x03100000u && t < toward;
+    if (__builtin_amdgcn_ballot_w64(!plain) == 0)
+        return __longlong_as_double((long long)((unsigned long long)((hi & 0x7ff00000u) - 0x03000000u) << 32));
+    return cm::min_step(t, toward);
+}
+CLODE_DEV float wave_min_step(float t, float toward)
+{
+    const unsigned int u = __float_as_uint(t);
+    const bool plain = u - 0x0a000000u < 0x7f000000u - 0x0a000000u && t < toward;
+    if (__builtin_amdgcn_ballot_w64(!plain) == 0)
+        return __uint_as_float((u & 0x7f800000u) - 0x09800000u);
+    return cm::min_step(t, toward);
+}
+#endif
 
 #if CLODE_PREC != 3
 // =====================================================================
@@ -310,25 +329,26 @@ CLODE_DEV realtype do_step(realtype &ti, realtype xi[], realtype k1[], const rea
 // when the step is done, either accepted or failed at hmin (state unchanged,
 // dt = hmin; the drivers do not distinguish the two, as the reference's do
 // not look at its -1 flag).
+//
+// Written without a branch but the copy of an accepted step: a lone wave pays
+// more for a region that some lanes skip (22 cycles) than for the selects.  A
+// stalled lane's trial is evaluated with the others' and dropped: its inputs
+// are those of its previous trial, so its aux values are too.  With exp's
+// shorter argument reduction (cm_math.h): lactotroph dopri5 in double, 65,536
+// members, 164.0 -> 148.4 ms over the three passes, one wave of 10 members
+// 3.51 -> 3.15 us a step; the flat loop also needs 57 instead of 170 reloads of
+// constants per trial, because no region boundary splits their live ranges.
 CLODE_DEV bool step_attempt(realtype &ti, realtype xi[], realtype k1[], const realtype pars[],
                             const SolverParamsR &sp, realtype &dt, const realtype t1,
                             realtype aux[], realtype wi[], RngData &rd, StepCtl &c)
 {
     realtype tNew, normErr, err[N_VAR], newxi[N_VAR], newk1[N_VAR];
-    realtype threshold = sp.abstol / sp.reltol;
-    realtype hmin = cm::min_step(ti, RCONST(1.1) * t1);  // 16 |fabs(nextafter(ti, 1.1 t1)) - ti|
-    if (!c.inStep) {
-        c.inStep = true;
-        c.noFailedSteps = true;
-        c.attempts = 0;
-        c.newDt = dt;
-    }
-    realtype newDt = fmin(fmax(c.newDt, hmin), sp.dtmax);
-    if ((!c.noFailedSteps && newDt == c.lastDt) || ++c.attempts > CLODE_MAX_ATTEMPTS) {
-        dt = hmin;  // stalled at hmin: the reference would retry this trial forever
-        c.inStep = false;
-        return true;
-    }
+    const realtype threshold = sp.abstol / sp.reltol;
+    const realtype hmin = wave_min_step(ti, RCONST(1.1) * t1);  // 16 |fabs(nextafter(ti, 1.1 t1)) - ti|
+    const bool retry = c.attempts != 0;
+    realtype newDt = fmin(fmax(dt, hmin), sp.dtmax);
+    // stalled at hmin: the reference would retry this trial forever
+    const bool stalled = (retry & (newDt == c.lastDt)) | (c.attempts >= CLODE_MAX_ATTEMPTS);
     c.lastDt = newDt;
     tNew = ti;
     for (int j = 0; j < N_VAR; j++) {
@@ -341,33 +361,27 @@ CLODE_DEV bool step_attempt(realtype &ti, realtype xi[], realtype k1[], const re
     normErr = ZERO;
     for (int j = 0; j < N_VAR; j++)
         normErr = fmax(fabs(err[j]), normErr);
-    // the factor both outcomes use, formed once for the whole wave:
-    // 0.8 (rtol/err)^(1/(p+1)) (the reference's pow(rtol/err, 1/(p+1)),
-    // here the division-free fixed root shared with the CPU oracle)
+    // the factor both outcomes use: 0.8 (rtol/err)^(1/(p+1)) (the reference's
+    // pow(rtol/err, 1/(p+1)), here the division-free fixed root shared with
+    // the CPU oracle)
     const realtype factor = RCONST(0.8) * cm::root<CLODE_ROOT_N>(sp.reltol / normErr);
-    if (normErr > sp.reltol) {
-        if (newDt <= hmin) {
-            dt = hmin;
-            c.inStep = false;
-            return true;
+    const bool rejected = normErr > sp.reltol;
+    const bool failed = stalled | (rejected & (newDt <= hmin));
+    const bool accepted = !(stalled | rejected);
+    const realtype shrunk = newDt * (retry ? RCONST(0.5) : fmax(CLODE_MAX_SHRINK, factor));
+    realtype grown = retry ? newDt : newDt * fmin(CLODE_MAX_GROW, factor);
+    grown = fmin(grown, t1 - tNew);
+    grown = fmin(fmax(grown, hmin), sp.dtmax);
+    dt = failed ? hmin : (rejected ? shrunk : grown);
+    c.attempts = failed | accepted ? 0 : c.attempts + 1;
+    if (accepted) {
+        ti = tNew;
+        for (int j = 0; j < N_VAR; j++) {
+            xi[j] = newxi[j];
+            k1[j] = newk1[j];
         }
-        newDt *= c.noFailedSteps ? fmax(CLODE_MAX_SHRINK, factor) : RCONST(0.5);
-        c.noFailedSteps = false;
-        c.newDt = newDt;
-        return false;
     }
-    if (c.noFailedSteps)
-        newDt *= fmin(CLODE_MAX_GROW, factor);
-    newDt = fmin(newDt, t1 - tNew);
-    newDt = fmin(fmax(newDt, hmin), sp.dtmax);
-    dt = newDt;
-    ti = tNew;
-    for (int j = 0; j < N_VAR; j++) {
-        xi[j] = newxi[j];
-        k1[j] = newk1[j];
-    }
-    c.inStep = false;
-    return true;
+    return failed | accepted;
 }
 #endif
 
@@ -586,19 +600,10 @@ CLODE_DEV bool step_attempt(double &ti, realtype xi[], realtype xc[], realtype k
 {
     double tNew, normErr;
     realtype err[N_VAR], newxi[N_VAR], newk1[N_VAR], dx[N_VAR];
-    double hmin = cm::min_step(ti, 1.1 * t1);  // 16 |fabs(nextafter(ti, 1.1 t1)) - ti|
-    if (!c.inStep) {
-        c.inStep = true;
-        c.noFailedSteps = true;
-        c.attempts = 0;
-        c.newDt = dt;
-    }
-    double newDt = fmin(fmax(c.newDt, hmin), dtmax);
-    if ((!c.noFailedSteps && newDt == c.lastDt) || ++c.attempts > CLODE_MAX_ATTEMPTS) {
-        dt = hmin;  // stalled at hmin (see CLODE_MAX_ATTEMPTS)
-        c.inStep = false;
-        return true;
-    }
+    const double hmin = wave_min_step(ti, 1.1 * t1);  // 16 |fabs(nextafter(ti, 1.1 t1)) - ti|
+    const bool retry = c.attempts != 0;
+    double newDt = fmin(fmax(dt, hmin), dtmax);
+    const bool stalled = (retry & (newDt == c.lastDt)) | (c.attempts >= CLODE_MAX_ATTEMPTS);
     c.lastDt = newDt;
     tNew = ti;
     for (int j = 0; j < N_VAR; j++) {
@@ -617,30 +622,24 @@ CLODE_DEV bool step_attempt(double &ti, realtype xi[], realtype xc[], realtype k
     const realtype q =
         fminf(fmaxf((realtype)reltol * __builtin_amdgcn_rcpf((realtype)normErr), 1.0e-30f), 1.0e30f);
     const double factor = (double)(0.8f * __builtin_amdgcn_exp2f(CLODE_EXPON * __builtin_amdgcn_logf(q)));
-    if (normErr > reltol) {
-        if (newDt <= hmin) {
-            dt = hmin;
-            c.inStep = false;
-            return true;
+    const bool rejected = normErr > reltol;
+    const bool failed = stalled | (rejected & (newDt <= hmin));
+    const bool accepted = !(stalled | rejected);
+    const double shrunk = newDt * (retry ? 0.5 : fmax(CLODE_MAX_SHRINK, factor));
+    double grown = retry ? newDt : newDt * fmin(CLODE_MAX_GROW, factor);
+    grown = fmin(grown, t1 - tNew);
+    grown = fmin(fmax(grown, hmin), dtmax);
+    dt = failed ? hmin : (rejected ? shrunk : grown);
+    c.attempts = failed | accepted ? 0 : c.attempts + 1;
+    if (accepted) {
+        ti = tNew;
+        for (int j = 0; j < N_VAR; j++) {
+            // newxi = xi + dx (rounded); redo the addition with compensation
+            kahan_add(xi[j], xc[j], dx[j]);
+            k1[j] = newk1[j];
         }
-        newDt *= c.noFailedSteps ? fmax(CLODE_MAX_SHRINK, factor) : 0.5;
-        c.noFailedSteps = false;
-        c.newDt = newDt;
-        return false;
     }
-    if (c.noFailedSteps)
-        newDt *= fmin(CLODE_MAX_GROW, factor);
-    newDt = fmin(newDt, t1 - tNew);
-    newDt = fmin(fmax(newDt, hmin), dtmax);
-    dt = newDt;
-    ti = tNew;
-    for (int j = 0; j < N_VAR; j++) {
-        // newxi = xi + dx (rounded); redo the addition with compensation
-        kahan_add(xi[j], xc[j], dx[j]);
-        k1[j] = newk1[j];
-    }
-    c.inStep = false;
-    return true;
+    return failed | accepted;
 }
 #endif
 

@@ -37,6 +37,40 @@
 
 namespace cm {
 
+// fmax and fmin of doubles without the compiler's quieting of operands.  In
+// the hardware's IEEE mode v_max_f64 returns a quiet NaN for a signalling one,
+// so the compiler first canonicalises every operand that it cannot trace to an
+// arithmetic result in the same block: loop-carried extrema and quotients cost
+// three instructions instead of one.  Every operand here is an arithmetic
+// result, never a signalling NaN.
+#if defined(__AMDGCN__)
+CM_FN double max_num(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+CM_FN double min_num(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+CM_FN double clamp_num(double a, double lo, double hi)  // lo, hi: uniform
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "s"(lo));
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(r), "s"(hi));
+    return r;
+}
+#else
+CM_FN double max_num(double a, double b) { return fmax(a, b); }
+CM_FN double min_num(double a, double b) { return fmin(a, b); }
+CM_FN double clamp_num(double a, double lo, double hi) { return fmin(fmax(a, lo), hi); }
+#endif
+CM_FN float max_num(float a, float b) { return fmaxf(a, b); }
+CM_FN float min_num(float a, float b) { return fminf(a, b); }
+
 // ---------------------------------------------------------------- double --
 CM_FN double exp(double x)
 {
@@ -48,8 +82,13 @@ CM_FN double exp(double x)
     const double log2e = 0x1.71547652b82fep+0;
     const double ln2hi = 0x1.62e42fefa39efp-1;
     const double ln2lo = 0x1.abc9e3b39803fp-56;
-    double xc = fmin(fmax(x, -746.0), 710.0);
-    double k = rint(xc * log2e);
+    double xc = clamp_num(x, -746.0, 710.0);
+    // k = x log2 e rounded to a whole number by adding 1.5 2^52, which also
+    // leaves k in the low bits of the sum (two instructions for the product,
+    // the rounding and the conversion to int)
+    const double shift = 0x1.8p52;
+    double ks = fma(xc, log2e, shift);
+    double k = ks - shift;
     double r = fma(-k, ln2hi, xc);
     r = fma(-k, ln2lo, r);
     // exp(r) = 1 + r + r^2 Q(r) on |r| <= ln2/2: Q of degree 9 interpolating
@@ -67,8 +106,15 @@ CM_FN double exp(double x)
     p = fma(p, r, 0x1.0000000000001p-1);
     p = fma(p, r, 1.0);
     p = fma(p, r, 1.0);
-    double y = ldexp(p, (int)k);
-    return (x == x) ? y : x;
+    unsigned long long kb, yb;
+    __builtin_memcpy(&kb, &ks, 8);
+    double y = ldexp(p, (int)(unsigned int)kb);
+    // NaN: the high half alone makes the result one
+    __builtin_memcpy(&yb, &y, 8);
+    const unsigned int hi = (x == x) ? (unsigned int)(yb >> 32) : 0x7ff80000u;
+    yb = ((unsigned long long)hi << 32) | (unsigned int)yb;
+    __builtin_memcpy(&y, &yb, 8);
+    return y;
 }
 
 CM_FN double log(double x)
@@ -277,6 +323,37 @@ CM_FN float root(float x)
 // exponent read and a scale instead of nextafter's integer sequence.  Other
 // arguments (t <= 0, subnormal, the largest finite value, a step downward,
 // NaN) take the formula itself.
+CM_FN double next_after(double x, double y)  // C's nextafter, inline on the device
+{
+    if (!(x == x) || !(y == y))
+        return x + y;
+    if (x == y)
+        return y;
+    unsigned long long u;
+    __builtin_memcpy(&u, &x, 8);
+    if (x == 0.0)
+        u = (y < 0.0 ? 0x8000000000000000ull : 0ull) + 1ull;
+    else
+        u = ((x < y) == (x > 0.0)) ? u + 1ull : u - 1ull;
+    __builtin_memcpy(&x, &u, 8);
+    return x;
+}
+CM_FN float next_after(float x, float y)
+{
+    if (!(x == x) || !(y == y))
+        return x + y;
+    if (x == y)
+        return y;
+    unsigned int u;
+    __builtin_memcpy(&u, &x, 4);
+    if (x == 0.0f)
+        u = (y < 0.0f ? 0x80000000u : 0u) + 1u;
+    else
+        u = ((x < y) == (x > 0.0f)) ? u + 1u : u - 1u;
+    __builtin_memcpy(&x, &u, 4);
+    return x;
+}
+
 CM_FN double min_step(double t, double toward)
 {
     if (t >= 0x1p-1022 && t < 0x1.fffffffffffffp+1023 && t < toward) {
@@ -284,7 +361,7 @@ CM_FN double min_step(double t, double toward)
         (void)frexp(t, &e);  // t = m 2^e, m in [1/2, 1): ilogb(t) = e - 1
         return ldexp(1.0, e - 49);
     }
-    return 16.0 * fabs(fabs(nextafter(t, toward)) - t);
+    return 16.0 * fabs(fabs(next_after(t, toward)) - t);
 }
 
 // float: spacing 2^(ilogb(t) - 23), so 16 spacings are 2^(ilogb(t) - 19)
@@ -295,7 +372,7 @@ CM_FN float min_step(float t, float toward)
         (void)frexpf(t, &e);
         return ldexpf(1.0f, e - 20);
     }
-    return 16.0f * fabsf(fabsf(nextafterf(t, toward)) - t);
+    return 16.0f * fabsf(fabsf(next_after(t, toward)) - t);
 }
 
 // ----------------------------------------------------------------- float --
