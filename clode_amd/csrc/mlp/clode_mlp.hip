@@ -54,6 +54,7 @@ constexpr int NLAYER = NHID + 1;
 
 typedef uint16_t bf16_t;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
@@ -299,22 +300,6 @@ __global__ void __launch_bounds__(256) mlp_gemm(const GemmArgs g)
     gemm_block<EPI, T>(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, smem);
 }
 
-// two independent products in one launch (a layer's weight gradient and its
-// input gradient): blocks [0, n1) are the first product's grid (gx1 x gy1 x
-// splits, x fastest), the rest the second's (gx2 wide); each block computes
-// exactly what it computes in a launch of its own
-template <int EPI1, int EPI2, int T>
-__global__ void __launch_bounds__(256) mlp_gemm_pair(const GemmArgs g1, int gx1, int gy1, int n1, const GemmArgs g2,
-                                                     int gx2)
-{
-    __shared__ __attribute__((aligned(16))) bf16_t smem[(Tile<T>::TM + Tile<T>::TN) * (Tile<T>::KC + KPAD)];
-    const int b = (int)blockIdx.x;
-    if (b < n1)
-        gemm_block<EPI1, T>(g1, b % gx1, (b / gx1) % gy1, b / (gx1 * gy1), smem);
-    else
-        gemm_block<EPI2, T>(g2, (b - n1) % gx2, (b - n1) / gx2, 0, smem);
-}
-
 // ---------------------------------------------------------------- encode
 // Fourier feature f of the input (x0, x1): sin and cos of
 // 2 pi (B[0][f] x0 + B[1][f] x1), rounded to BF16
@@ -386,6 +371,41 @@ __host__ __device__ inline bool head_keeps(unsigned long long sample, int head)
 constexpr int PADROWS = (NOUTP - NOUT) / NHEAD;  // transposed padding rows each head thread clears
 static_assert(PADROWS * NHEAD == NOUTP - NOUT, "padding rows split evenly over the heads");
 
+// one (row, head): its loss into l, the gradient of its 18 outputs into d
+__device__ __attribute__((always_inline)) inline void loss_row(const float *zh, bool kept, float t0, float t1, int y,
+                                                               float inv_n, bf16_t (&d)[HW], float &l)
+{
+    if (!kept) {
+#pragma unroll
+        for (int c = 0; c < HW; ++c)
+            d[c] = 0;
+        return;
+    }
+    const float e0 = zh[0] - t0, e1 = zh[1] - t1;
+    l += e0 * e0 + e1 * e1;
+    d[0] = f2bf(2.f * e0 * inv_n);
+    d[1] = f2bf(2.f * e1 * inv_n);
+    float mx = zh[2];
+#pragma unroll
+    for (int c = 1; c < NCLS; ++c)
+        mx = fmaxf(mx, zh[2 + c]);
+    // each class's exponential once, for the sum and the gradient
+    float ex[NCLS];
+    float se = 0.f, zy = zh[2];
+#pragma unroll
+    for (int c = 0; c < NCLS; ++c) {
+        ex[c] = __expf(zh[2 + c] - mx);
+        se += ex[c];
+        zy = c == y ? zh[2 + c] : zy;
+    }
+    l += (mx + __logf(se)) - zy;
+#pragma unroll
+    for (int c = 0; c < NCLS; ++c) {
+        const float p = ex[c] / se;
+        d[2 + c] = f2bf((p - (c == y ? 1.f : 0.f)) * inv_n);
+    }
+}
+
 __global__ void __launch_bounds__(256) mlp_loss(const float *Zh, int n, const float *T, const int *cls,
                                                 const unsigned long long *ids, float inv_n, bf16_t *dOut,
                                                 bf16_t *dOutT, int ldt, float *loss)
@@ -395,36 +415,9 @@ __global__ void __launch_bounds__(256) mlp_loss(const float *Zh, int n, const fl
     float l = 0.f;
     if (t < (long long)NHEAD * n) {
         const int h = (int)(t / n), i = (int)(t % n);
-        const float *zh = Zh + (long long)i * NOUTP + h * HW;
         bf16_t d[HW];
         const unsigned long long id = ids ? ids[i] : (unsigned long long)i;
-        if (!head_keeps(id, h)) {
-            for (int c = 0; c < HW; ++c)
-                d[c] = 0;
-        } else {
-            const float e0 = zh[0] - T[2 * i], e1 = zh[1] - T[2 * i + 1];
-            l += e0 * e0 + e1 * e1;
-            d[0] = f2bf(2.f * e0 * inv_n);
-            d[1] = f2bf(2.f * e1 * inv_n);
-            float mx = zh[2];
-            for (int c = 1; c < NCLS; ++c)
-                mx = fmaxf(mx, zh[2 + c]);
-            // each class's exponential once, for the sum and the gradient
-            float ex[NCLS];
-            float se = 0.f;
-#pragma unroll
-            for (int c = 0; c < NCLS; ++c) {
-                ex[c] = __expf(zh[2 + c] - mx);
-                se += ex[c];
-            }
-            const int y = cls[i];
-            l += (mx + __logf(se)) - zh[2 + y];
-#pragma unroll
-            for (int c = 0; c < NCLS; ++c) {
-                const float p = ex[c] / se;
-                d[2 + c] = f2bf((p - (c == y ? 1.f : 0.f)) * inv_n);
-            }
-        }
+        loss_row(Zh + (long long)i * NOUTP + h * HW, head_keeps(id, h), T[2 * i], T[2 * i + 1], cls[i], inv_n, d, l);
         bf16_t *dh = dOut + (long long)i * NOUTP + h * HW;
         for (int c = 0; c < HW; ++c) {
             dh[c] = d[c];
@@ -481,20 +474,61 @@ __global__ void __launch_bounds__(256) mlp_layer_grads(const float *part, int sp
 
 // layer table for the Adam kernels: weights of layer l occupy
 // [woff, woff + in * out) as Wt[out][in], its biases the out entries after
-// them; the transposed BF16 copy keeps W[in][out] at the same offsets
+// them
 struct LayerTable {
     long long woff[NLAYER];
     int in[NLAYER], out[NLAYER];
 };
 
+// The BF16 copies of the weights that the products read, all at the layer's
+// weight offset: Wt[out][in], W[in][out], and both again in fragment order.
+struct WeightCopies {
+    bf16_t *w, *wT, *f, *fT;
+};
+
+// Fragment order of a product's B operand, rows n of K entries: the 16 x 32
+// block of rows 16 nb .. and entries 32 kb .. is 512 consecutive values, the 8
+// of lane (k / 8 % 4) * 16 + n % 16 together, so that a wave's load of one
+// fragment is 1 KB in a row.  From Wt[out][in] the same load touches 16 rows, a
+// different one in every consecutive lane.
+__device__ inline int frag_at(int n, int k, int K)
+{
+    return ((n >> 4) * (K >> 5) + (k >> 5)) * 512 + (((k >> 3) & 3) * 16 + (n & 15)) * 8 + (k & 7);
+}
+
+// parameter i in the copies (a bias only at its place in the first)
+__device__ __forceinline__ void put_weight(const WeightCopies &c, const LayerTable &lt, long long i, float v)
+{
+    const bf16_t b16 = f2bf(v);
+    c.w[i] = b16;
+    int l = 0;
+    while (l < NLAYER - 1 && i >= lt.woff[l + 1])
+        ++l;
+    const int r = (int)(i - lt.woff[l]), in = lt.in[l], out = lt.out[l];
+    if (r >= in * out)
+        return;
+    const int o = r / in, k = r % in;
+    c.wT[lt.woff[l] + k * out + o] = b16;
+    c.f[lt.woff[l] + frag_at(o, k, in)] = b16;
+    c.fT[lt.woff[l] + frag_at(k, o, out)] = b16;
+}
+
+__global__ void __launch_bounds__(256) mlp_put_weights(const float *p, const WeightCopies c, const LayerTable lt,
+                                                       long long n)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        put_weight(c, lt, i, p[i]);
+}
+
 struct AdamStep {
     float lr, b1, b2, eps, c1, c2;
 };
 
-// Adam (Kingma & Ba 2015) on one FP32 master parameter, refreshing both BF16
+// Adam (Kingma & Ba 2015) on one FP32 master parameter, refreshing the BF16
 // copies of the weights
-__device__ __forceinline__ void adam_update(long long i, float gi, float *p, float *m1, float *m2, bf16_t *pbf,
-                                            bf16_t *pbfT, const LayerTable &lt, const AdamStep &as)
+__device__ __forceinline__ void adam_update(long long i, float gi, float *p, float *m1, float *m2,
+                                            const WeightCopies &wc, const LayerTable &lt, const AdamStep &as)
 {
     const float a = as.b1 * m1[i] + (1.f - as.b1) * gi;
     const float b = as.b2 * m2[i] + (1.f - as.b2) * gi * gi;
@@ -502,27 +536,19 @@ __device__ __forceinline__ void adam_update(long long i, float gi, float *p, flo
     m2[i] = b;
     const float v = p[i] - as.lr * (a * as.c1) / (sqrtf(b * as.c2) + as.eps);
     p[i] = v;
-    const bf16_t b16 = f2bf(v);
-    pbf[i] = b16;
-    for (int l = 0; l < NLAYER; ++l) {
-        const long long r = i - lt.woff[l];
-        if (r >= 0 && r < (long long)lt.in[l] * lt.out[l]) {
-            const int o = (int)(r / lt.in[l]), k = (int)(r % lt.in[l]);
-            pbfT[lt.woff[l] + (long long)k * lt.out[l] + o] = b16;
-        }
-    }
+    put_weight(wc, lt, i, v);
 }
 
 // Adam from a finished gradient vector g; frozen entries (mask 0: head
 // padding) stay put
 __global__ void __launch_bounds__(256) mlp_adam(float *p, const float *g, float *m1, float *m2, const uint8_t *mask,
-                                                bf16_t *pbf, bf16_t *pbfT, const LayerTable lt, long long n,
+                                                const WeightCopies wc, const LayerTable lt, long long n,
                                                 const AdamStep as)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || !mask[i])
         return;
-    adam_update(i, g[i], p, m1, m2, pbf, pbfT, lt, as);
+    adam_update(i, g[i], p, m1, m2, wc, lt, as);
 }
 
 // Adam that also finishes the gradient, in place of the per-layer reduction
@@ -541,8 +567,8 @@ struct GradSources {
     int n, ld;
 };
 
-__global__ void __launch_bounds__(256) mlp_adam_sum(float *p, float *m1, float *m2, const uint8_t *mask, bf16_t *pbf,
-                                                    bf16_t *pbfT, const LayerTable lt, long long n, int wblocks,
+__global__ void __launch_bounds__(256) mlp_adam_sum(float *p, float *m1, float *m2, const uint8_t *mask,
+                                                    const WeightCopies wc, const LayerTable lt, long long n, int wblocks,
                                                     const GradSources gs, const AdamStep as)
 {
     if ((int)blockIdx.x < wblocks) {
@@ -557,7 +583,7 @@ __global__ void __launch_bounds__(256) mlp_adam_sum(float *p, float *m1, float *
         float s = 0.f;
         for (int z = 0; z < gs.splits; ++z)
             s += gs.part[(long long)z * gs.pstride + i];
-        adam_update(i, s, p, m1, m2, pbf, pbfT, lt, as);
+        adam_update(i, s, p, m1, m2, wc, lt, as);
         return;
     }
     __shared__ float red[256];
@@ -566,6 +592,9 @@ __global__ void __launch_bounds__(256) mlp_adam_sum(float *p, float *m1, float *
         c -= lt.out[l];
         ++l;
     }
+    const long long i = lt.woff[l] + (long long)lt.in[l] * lt.out[l] + c;
+    if (!mask[i])
+        return;  // head padding: its gradient rows are not formed
     const bf16_t *dzt = gs.dzt[l];
     float s = 0.f;
     for (int m = threadIdx.x; m < gs.n; m += blockDim.x)
@@ -577,9 +606,8 @@ __global__ void __launch_bounds__(256) mlp_adam_sum(float *p, float *m1, float *
             red[threadIdx.x] += red[threadIdx.x + k];
         __syncthreads();
     }
-    const long long i = lt.woff[l] + (long long)lt.in[l] * lt.out[l] + c;
-    if (threadIdx.x == 0 && mask[i])
-        adam_update(i, red[0], p, m1, m2, pbf, pbfT, lt, as);
+    if (threadIdx.x == 0)
+        adam_update(i, red[0], p, m1, m2, wc, lt, as);
 }
 
 // minibatch gather: row r of the batch is sample perm[r] of the training
@@ -741,6 +769,7 @@ thread_local std::string g_err;
 // layer the same bytes hold the FP32 head outputs [SROWS][ZPITCH].
 constexpr int SROWS = 128;         // cells per workgroup
 constexpr int ZPITCH = NOUT + 1;   // row pitch of the head outputs (floats)
+constexpr int HBLK = (NOUT + 15) / 16;  // column blocks of the heads that hold used columns
 static_assert(SROWS * ZPITCH * 4 <= SROWS * H * 2, "head outputs fit in the activation buffer");
 static_assert(SROWS == 8 * 16 && H == 4 * 64 && NOUTP == 4 * 32, "wave tiling");
 
@@ -787,13 +816,13 @@ __device__ __attribute__((always_inline)) inline void screen_product(const bf16_
     bf16x8 b[NB], bn[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-        b[j] = *(const bf16x8 *)(W + (long long)(n0 + j * 16 + r) * K + kq);
+        b[j] = *(const bf16x8 *)(W + ((n0 / 16 + j) * NKS) * 512 + lane * 8);
 #pragma unroll 1
     for (int ks = 0; ks < NKS; ++ks) {
         if (ks + 1 < NKS) {
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-                bn[j] = *(const bf16x8 *)(W + (long long)(n0 + j * 16 + r) * K + (ks + 1) * TK + kq);
+                bn[j] = *(const bf16x8 *)(W + ((n0 / 16 + j) * NKS + ks + 1) * 512 + lane * 8);
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -885,6 +914,245 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
     }
 }
 
+// ---------------------------------------------------------------- fused training pass
+// One launch for everything of an optimizer step that runs row by row: gather
+// and encode, the four hidden layers, the heads, the loss, and the input
+// gradients back to the first layer.  A workgroup of 8 waves takes 16 rows of
+// the minibatch; activations and gradients stay in LDS (two 8 KiB tiles, one
+// barrier per layer), SiLU' stays in the registers of the lane that needs it
+// again (a lane forms the same elements of a layer forward and backward), and
+// each wave's weight fragments of the next product are loaded while the current
+// one runs.  Only the transposed operands of the weight-gradient products leave
+// the CU.
+// What bounds it is the chain of nine products, each waiting for the one
+// before: 17 us with 4 workgroups, 21 us with 128 (2048 rows), 23 us with 256;
+// past one workgroup per CU the weights' way from L2, 1 MB per workgroup at
+// 64 B per cycle, 17 us per 256 workgroups.  An optimizer step's three launches
+// take 40 us at 2048 rows and 29 us at 64; the thirteen that this replaces
+// (gather, five forward products, loss, five backward pairs, optimizer) took
+// 79 us and 58 us, each waiting for a few hundred workgroups to start and drain.
+// K order and epilogue arithmetic are those of gemm_block, so the weights
+// after training are the same bits.
+constexpr int FROWS = 16;    // rows per workgroup
+constexpr int FWAVES = 8;    // waves per workgroup, 32 columns each
+constexpr int FKH = 96;      // head gradient columns that can be nonzero, in whole K steps
+static_assert(FWAVES * 32 == H && HBLK <= FWAVES && NOUT <= FKH && FKH % TK == 0, "fused training tiling");
+
+struct FusedStep {
+    const unsigned int *perm;  // this minibatch's samples
+    int nb, ldt;
+    const float *Xa, *Ta;
+    const int *Ca;
+    const float *Bff;
+    const bf16_t *W[NLAYER];   // Wt[out][in] and
+    const bf16_t *WT[NLAYER];  // W[in][out], in fragment order
+    const float *bias[NLAYER];
+    bf16_t *A0t, *Yt[NHID], *dYt[NHID], *dOutT;  // [width][ldt]
+    float inv_n;
+    float *loss;
+};
+
+// weight fragments of NB column blocks from block nb0 for the first K of KW entries
+template <int K, int NB, int KW = K>
+__device__ __attribute__((always_inline)) inline void fused_load(const bf16_t *__restrict__ W, int nb0, int lane,
+                                                                 bf16x8 (&b)[K / TK][NB])
+{
+#pragma unroll
+    for (int ks = 0; ks < K / TK; ++ks)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            b[ks][j] = *(const bf16x8 *)(W + ((nb0 + j) * (KW / TK) + ks) * 512 + lane * 8);
+}
+
+template <int K, int NB>
+__device__ __attribute__((always_inline)) inline void fused_product(const bf16_t *act, const bf16x8 (&b)[K / TK][NB],
+                                                                    int lane, f32x4 (&acc)[NB])
+{
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+        acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < K / TK; ++ks) {
+        const bf16x8 a = *(const bf16x8 *)&act[sw(lane & 15, ks * TK + (lane >> 4) * 8)];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[ks][j], acc[j], 0, 0, 0);
+    }
+}
+
+// four rows ml .. ml + 3 of column n: into the activation tile, and at dst in
+// the transposed copy, whose rows past the minibatch are padding
+__device__ __attribute__((always_inline)) inline void fused_put(bf16_t *act, int ml, int n, const bf16x4 &y, bf16_t *dst)
+{
+    union {
+        bf16x4 v;
+        bf16_t e[4];
+    } u = {y};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        act[sw(ml + q, n)] = u.e[q];
+    *(bf16x4 *)dst = y;
+}
+
+__global__ void __launch_bounds__(FWAVES * 64) mlp_fused_step(const FusedStep s)
+{
+    __shared__ __attribute__((aligned(16))) bf16_t act[2][FROWS * H];
+    __shared__ float zh[FROWS * ZPITCH];
+    __shared__ float bias[NHID * H + NOUT];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // 8 consecutive workgroups are on 8 XCDs: each XCD takes consecutive rows,
+    // which share the lines of the transposed copies
+    const int per = (int)(gridDim.x >> 3);
+    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    const int r0 = tile * FROWS;                       // the workgroup's rows of the minibatch
+    if (r0 >= s.nb)
+        return;
+    const int ml = (lane >> 4) * 4, m = r0 + ml;       // the lane's four output rows
+    const int n0 = wave * 32, c0 = n0 + (lane & 15);   // the wave's columns, the lane's first
+    // everything that is read from memory apart from weights comes first: a
+    // later load would wait for the prefetched weights and the stores before it
+    const int rr = t & 15, row = r0 + rr;
+    const unsigned int id = s.perm[row < s.nb ? row : s.nb - 1];
+    const float x0 = s.Xa[2 * (size_t)id], x1 = s.Xa[2 * (size_t)id + 1];
+    const float t0 = s.Ta[2 * (size_t)id], t1 = s.Ta[2 * (size_t)id + 1];
+    const int cls = s.Ca[id];
+#pragma unroll
+    for (int l = 0; l < NHID; l += 2) {
+        const int l1 = l + (t >> 8), n = t & 255;
+        bias[l1 * H + n] = s.bias[l1][n];
+    }
+    if (t < NOUT)
+        bias[NHID * H + t] = s.bias[NHID][t];
+    bf16x8 b0[1][2], ba[H / TK][2], bb[H / TK][2];
+    fused_load<D0, 2>(s.W[0], n0 / 16, lane, b0);
+    fused_load<H, 2>(s.W[1], n0 / 16, lane, ba);
+    if (t < FROWS * NFF) {
+        const int f = t >> 4;
+        bf16_t sv, cv;
+        encode_pair(x0, x1, f, s.Bff, sv, cv);
+        act[0][sw(rr, 2 * f)] = sv;
+        act[0][sw(rr, 2 * f + 1)] = cv;
+        s.A0t[(long long)(2 * f) * s.ldt + row] = sv;
+        s.A0t[(long long)(2 * f + 1) * s.ldt + row] = cv;
+    }
+    __syncthreads();
+    f32x4 D[NHID][2];  // SiLU'(z), for the way back
+    auto hidden = [&](int l, f32x4 (&acc)[2], bf16_t *out) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = c0 + j * 16;
+            const float bj = bias[l * H + n];
+            bf16x4 y;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v = acc[j][q];
+                v += bj;
+                const float sg = sigm(v);
+                D[l][j][q] = sg * (1.0f + v * (1.0f - sg));
+                y[q] = (__bf16)(v * sg);
+            }
+            fused_put(out, ml, n, y, s.Yt[l] + (long long)n * s.ldt + m);
+        }
+        __syncthreads();
+    };
+    f32x4 acc[2];
+    fused_product<D0, 2>(act[0], b0, lane, acc);
+    hidden(0, acc, act[1]);
+    fused_load<H, 2>(s.W[2], n0 / 16, lane, bb);
+    fused_product<H, 2>(act[1], ba, lane, acc);
+    hidden(1, acc, act[0]);
+    fused_load<H, 2>(s.W[3], n0 / 16, lane, ba);
+    fused_product<H, 2>(act[0], bb, lane, acc);
+    hidden(2, acc, act[1]);
+    // heads: one 16-column block on each of the first waves
+    bf16x8 bh[H / TK][1];
+    const int hb = wave < HBLK ? wave : 0;
+    fused_load<H, 1>(s.W[NHID], hb, lane, bh);
+    fused_product<H, 2>(act[1], ba, lane, acc);
+    hidden(3, acc, act[0]);
+    bf16x8 bg[FKH / TK][2];
+    fused_load<FKH, 2, NOUTP>(s.WT[NHID], n0 / 16, lane, bg);
+    fused_load<H, 2>(s.WT[3], n0 / 16, lane, bb);
+    {
+        f32x4 az[1];
+        fused_product<H, 1>(act[0], bh, lane, az);
+        const int n = hb * 16 + (lane & 15);
+        if (wave < HBLK && n < NOUT) {
+            const float bj = bias[NHID * H + n];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v = az[0][q];
+                v += bj;
+                zh[(ml + q) * ZPITCH + n] = v;
+            }
+        }
+    }
+    __syncthreads();
+    // loss and head gradient, one lane per (row, head), by the first wave; the
+    // others clear the gradient tile's columns past the heads
+    if (wave == 0) {
+        const int h = lane >> 4;
+        float l = 0.f;
+        bf16_t d[HW];
+        loss_row(zh + rr * ZPITCH + h * HW, row < s.nb && head_keeps(id, h), t0, t1, cls, s.inv_n, d, l);
+#pragma unroll
+        for (int c = 0; c < HW; ++c) {
+            act[1][sw(rr, h * HW + c)] = d[c];
+            s.dOutT[(long long)(h * HW + c) * s.ldt + row] = d[c];
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+            l += __shfl_xor(l, o);
+        if (lane == 0)
+            atomicAdd(s.loss, l * s.inv_n);
+    } else if (t < 64 + FROWS * (FKH - NOUT)) {
+        const int e = t - 64;
+        act[1][sw(e & 15, NOUT + (e >> 4))] = 0;
+    }
+    __syncthreads();
+    auto back = [&](int l, f32x4 (&g)[2], bf16_t *out) __attribute__((always_inline)) {  // into layer l's output gradient
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = c0 + j * 16;
+            bf16x4 y;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                y[q] = (__bf16)(g[j][q] * D[l][j][q]);
+            fused_put(out, ml, n, y, s.dYt[l] + (long long)n * s.ldt + m);
+        }
+        __syncthreads();
+    };
+    fused_product<FKH, 2>(act[1], bg, lane, acc);
+    back(3, acc, act[0]);
+    fused_load<H, 2>(s.WT[2], n0 / 16, lane, ba);
+    fused_product<H, 2>(act[0], bb, lane, acc);
+    back(2, acc, act[1]);
+    fused_load<H, 2>(s.WT[1], n0 / 16, lane, bb);
+    fused_product<H, 2>(act[1], ba, lane, acc);
+    back(1, acc, act[0]);
+    fused_product<H, 2>(act[0], bb, lane, acc);
+    back(0, acc, act[1]);
+}
+
+// every layer's weight-gradient product in one launch: blocks [first[l],
+// first[l + 1]) are layer l's grid, x fastest
+struct WgradAll {
+    GemmArgs g[NLAYER];
+    int gx[NLAYER], gy[NLAYER], first[NLAYER + 1];
+};
+
+template <int T>
+__global__ void __launch_bounds__(256) mlp_wgrad_all(const WgradAll a)
+{
+    __shared__ __attribute__((aligned(16))) bf16_t smem[(Tile<T>::TM + Tile<T>::TN) * (Tile<T>::KC + KPAD)];
+    const int b = (int)blockIdx.x;
+    int l = 0;
+    while (b >= a.first[l + 1])
+        ++l;
+    const int k = b - a.first[l];
+    gemm_block<EPI_WGRAD, T>(a.g[l], k % a.gx[l], k / a.gx[l] % a.gy[l], k / (a.gx[l] * a.gy[l]), smem);
+}
+
 struct MlpError : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
@@ -953,9 +1221,9 @@ struct clode_mlp {
     float tmean[2] = {0, 0}, tstd[2] = {1, 1};
     Dev<float> p, g, m1, m2, dBff, dT, dtm;
     Dev<uint8_t> mask;
-    Dev<bf16_t> pbf, pbfT;  // BF16 weights Wt[out][in] and W[in][out]
+    Dev<bf16_t> pbf, pbfT, pbfF, pbfTF;  // the WeightCopies
     // activations for a chunk of rows, and transposed copies [width][ldt]
-    // (ldt = rows rounded up to 8) for the weight-gradient products
+    // (ldt = rows rounded up to 16) for the weight-gradient products
     Dev<bf16_t> A0, Y[NHID], dY[NHID], dOut;
     Dev<bf16_t> A0t, Yt[NHID], dYt[NHID], dOutT;
     Dev<float> Z[NHID], Zh, X, T, loss, wsp;
@@ -967,24 +1235,45 @@ struct clode_mlp {
     size_t rows = 0;
     unsigned char *stage = nullptr;  // this device's static scratch (no-allocation screening)
 
+    WeightCopies copies() const { return {pbf.p, pbfT.p, pbfF.p, pbfTF.p}; }
+    LayerTable table() const
+    {
+        LayerTable lt;
+        for (int l = 0; l < NLAYER; ++l) {
+            lt.woff[l] = (long long)L[l].woff;
+            lt.in[l] = L[l].in;
+            lt.out[l] = L[l].out;
+        }
+        return lt;
+    }
+
+    // the transposed operands of the weight gradients (all that a fused
+    // training pass leaves in memory)
+    void ensureTransposed(size_t n)
+    {
+        const size_t nt = (n + FROWS - 1) / FROWS * FROWS;
+        A0t.alloc(nt * D0);
+        for (int l = 0; l < NHID; ++l) {
+            Yt[l].alloc(nt * H);
+            dYt[l].alloc(nt * H);
+        }
+        dOutT.alloc(nt * NOUTP);
+    }
+
     void ensureRows(size_t n)
     {
         if (n <= rows)
             return;
-        const size_t nt = (n + 7) & ~(size_t)7;
+        ensureTransposed(n);
         A0.alloc(n * D0);
-        A0t.alloc(nt * D0);
         for (int l = 0; l < NHID; ++l) {
             Y[l].alloc(n * H);
             dY[l].alloc(n * H);
-            Yt[l].alloc(nt * H);
-            dYt[l].alloc(nt * H);
             Z[l].alloc(n * H);
         }
         dOut.alloc(n * NOUTP);
         // the loss kernel never writes the padding columns: they stay zero
         check(hipMemsetAsync(dOut.p, 0, n * NOUTP * sizeof(bf16_t), stream), "hipMemsetAsync");
-        dOutT.alloc(nt * NOUTP);
         Zh.alloc(n * NOUTP);
         X.alloc(n * 2);
         T.alloc(n * 2);
@@ -1035,28 +1324,9 @@ void gemm(clode_mlp *h, int epi, const GemmArgs &a)
     }
 }
 
-// a layer's weight gradient w (split-K) and input gradient d (x SiLU') in
-// one launch when both use 32 x 32 tiles (the training minibatches), as two
-// launches otherwise; the same products either way
-void gemm_pair(clode_mlp *h, const GemmArgs &w, const GemmArgs &d)
-{
-    if (tile_for(h, w) != 32 || tile_for(h, d) != 32) {
-        gemm(h, EPI_WGRAD, w);
-        gemm(h, EPI_BWD_DSILU, d);
-        return;
-    }
-    const int gx1 = (w.N + 31) / 32, gy1 = (w.M + 31) / 32;
-    const int sp1 = w.ksplit > 0 ? (w.K + w.ksplit - 1) / w.ksplit : 1;
-    const int gx2 = (d.N + 31) / 32, gy2 = (d.M + 31) / 32;
-    const int n1 = gx1 * gy1 * sp1;
-    hipLaunchKernelGGL((mlp_gemm_pair<EPI_WGRAD, EPI_BWD_DSILU, 32>), dim3((unsigned int)(n1 + gx2 * gy2)),
-                       dim3(256), 0, h->stream, w, gx1, gy1, n1, d, gx2);
-    check(hipGetLastError(), "mlp_gemm_pair launch");
-}
-
 GemmArgs ga() { GemmArgs a; std::memset(&a, 0, sizeof(a)); return a; }
 
-inline int ldT(int n) { return (n + 7) & ~7; }
+inline int ldT(int n) { return (n + FROWS - 1) / FROWS * FROWS; }
 
 constexpr int KSPLIT_MAX = 32;    // partial products per weight gradient
 constexpr int KSPLIT_ROWS = 256;  // rows per partial product (at least)
@@ -1093,62 +1363,42 @@ void forward(clode_mlp *h, int n, bool train = false)
     gemm(h, EPI_FWD_LINEAR, a);
 }
 
+// layer l's weight gradient from the transposed operands of n rows, as split-K
+// partial products cstride apart: dWt[o][i] = sum_m dz[m][o] x[m][i] =
+// sum_m dzt[o][m] xt[i][m], the batch (the reduction) split so that the product
+// has enough workgroups
+GemmArgs wgrad_args(clode_mlp *h, int l, int n, const bf16_t *dzt, float *Cout, long long cstride, int *splits_used)
+{
+    const Layer &Ly = h->L[l];
+    const int lt = ldT(n);
+    GemmArgs w = ga();
+    w.M = Ly.out; w.N = Ly.in; w.K = n;
+    w.A = dzt; w.lda_m = lt; w.lda_k = 1;
+    w.B = l > 0 ? h->Yt[l - 1].p : h->A0t.p; w.ldb_k = 1; w.ldb_n = lt;
+    const int splits = std::max(1, std::min(KSPLIT_MAX, n / KSPLIT_ROWS));
+    w.ksplit = ((n + splits - 1) / splits + TK - 1) / TK * TK;
+    *splits_used = (n + w.ksplit - 1) / w.ksplit;
+    w.Cout = Cout; w.ldc = Ly.in; w.cstride = cstride;
+    return w;
+}
+
 // backward from h->dOut / h->dOutT (BF16) into h->g; every product reads
-// operands that are contiguous along its reduction index.  With gs (the
-// training loop) the split-K partial weight gradients of every layer stay in
-// h->wall (split z of parameter i at z * nparam + i) and the sums, with the
-// bias gradients, are left to the optimizer launch (mlp_adam_sum); gs
-// receives where they are.  Returns nothing to sum otherwise.
-void backward(clode_mlp *h, int n, GradSources *gs = nullptr)
+// operands that are contiguous along its reduction index
+void backward(clode_mlp *h, int n)
 {
     const int lt = ldT(n);
     const bf16_t *dz = h->dOut.p, *dzt = h->dOutT.p;
     int nout = NOUTP;
     for (int l = NHID; l >= 0; --l) {
         const Layer &Ly = h->L[l];
-        const bf16_t *xt = l > 0 ? h->Yt[l - 1].p : h->A0t.p;
-        // dWt[o][i] = sum_m dz[m][o] x[m][i] = sum_m dzt[o][m] xt[i][m]
-        // split the batch (the reduction) so that the product has enough
-        // workgroups, then sum the partial products in a fixed order
-        GemmArgs w = ga();
-        w.M = Ly.out; w.N = Ly.in; w.K = n;
-        w.A = dzt; w.lda_m = lt; w.lda_k = 1;
-        w.B = xt; w.ldb_k = 1; w.ldb_n = lt;
-        const int splits = std::max(1, std::min(KSPLIT_MAX, n / KSPLIT_ROWS));
-        w.ksplit = ((n + splits - 1) / splits + TK - 1) / TK * TK;
-        const int used = (n + w.ksplit - 1) / w.ksplit;
+        // the partial products are summed in a fixed order
+        int used = 0;
         const long long count = (long long)Ly.out * Ly.in;
-        if (gs) {
-            w.Cout = h->wall.p + Ly.woff; w.ldc = Ly.in; w.cstride = (long long)h->nparam;
-            gs->splits = used;
-            gs->dzt[l] = dzt;
-            if (l == 0) {
-                gemm(h, EPI_WGRAD, w);
-                break;
-            }
-            // the weight gradient and the input gradient read the same
-            // output gradient and nothing the other writes: one launch
-            GemmArgs d = ga();
-            d.M = n; d.N = Ly.in; d.K = Ly.out;
-            d.A = dz; d.lda_m = nout; d.lda_k = 1;
-            d.B = h->pbfT.p + Ly.woff; d.ldb_k = 1; d.ldb_n = Ly.out;
-            d.Zin = h->Z[l - 1].p; d.ldz = H;
-            d.Yout = h->dY[l - 1].p; d.ldy = H;
-            d.YTout = h->dYt[l - 1].p; d.ldt = lt;
-            gemm_pair(h, w, d);
-            dz = h->dY[l - 1].p;
-            dzt = h->dYt[l - 1].p;
-            nout = H;
-            continue;
-        } else {
-            w.Cout = h->wsp.p; w.ldc = Ly.in; w.cstride = count;
-            gemm(h, EPI_WGRAD, w);
-            const int sum_blocks = (int)((count + 255) / 256);
-            hipLaunchKernelGGL(mlp_layer_grads, dim3((unsigned int)(sum_blocks + Ly.out)), dim3(256), 0, h->stream,
-                               h->wsp.p, used, count, h->g.p + Ly.woff, sum_blocks, dzt, n, Ly.out, lt,
-                               h->g.p + Ly.boff);
-            check(hipGetLastError(), "mlp_layer_grads launch");
-        }
+        gemm(h, EPI_WGRAD, wgrad_args(h, l, n, dzt, h->wsp.p, count, &used));
+        const int sum_blocks = (int)((count + 255) / 256);
+        hipLaunchKernelGGL(mlp_layer_grads, dim3((unsigned int)(sum_blocks + Ly.out)), dim3(256), 0, h->stream,
+                           h->wsp.p, used, count, h->g.p + Ly.woff, sum_blocks, dzt, n, Ly.out, lt, h->g.p + Ly.boff);
+        check(hipGetLastError(), "mlp_layer_grads launch");
         if (l == 0)
             break;
         // dY[l-1][m][i] = (sum_o dz[m][o] W[i][o]) * silu'(Z[l-1][m][i])
@@ -1164,6 +1414,46 @@ void backward(clode_mlp *h, int n, GradSources *gs = nullptr)
         dzt = h->dYt[l - 1].p;
         nout = H;
     }
+}
+
+// One training step's row-wise pass and weight-gradient products, two launches.
+// The partial weight gradients of every layer stay in h->wall (split z of
+// parameter i at z * nparam + i); gs receives where they and the transposed
+// output gradients are, for mlp_adam_sum.
+void fused_step(clode_mlp *h, const FusedStep &f, GradSources &gs)
+{
+    hipLaunchKernelGGL(mlp_fused_step, dim3((unsigned int)((f.nb + 8 * FROWS - 1) / (8 * FROWS) * 8)), dim3(FWAVES * 64), 0, h->stream,
+                       f);
+    check(hipGetLastError(), "mlp_fused_step launch");
+    WgradAll a;
+    int blocks = 0, tiles64 = 0;
+    gs.part = h->wall.p;
+    gs.pstride = (long long)h->nparam;
+    gs.n = f.nb;
+    gs.ld = f.ldt;
+    for (int l = 0; l < NLAYER; ++l) {
+        gs.dzt[l] = l < NHID ? h->dYt[l].p : h->dOutT.p;
+        a.g[l] = wgrad_args(h, l, f.nb, gs.dzt[l], h->wall.p + h->L[l].woff, gs.pstride, &gs.splits);
+        if (l == NHID)
+            a.g[l].M = NOUT;  // the padding's gradients are not used
+        tiles64 += ((a.g[l].N + 63) / 64) * ((a.g[l].M + 63) / 64) * gs.splits;
+    }
+    // 32 x 32 tiles until 64 x 64 ones fill every CU twice: a step took 35.4
+    // and 37.7 us with them at 1000 rows (180 tiles of 64 x 64), the same at
+    // 2048 (480), 53.0 and 51.1 at 4096 (960), 175 and 168 at 16384
+    const int tile = tiles64 < 2 * h->cus ? 32 : 64;
+    for (int l = 0; l < NLAYER; ++l) {
+        a.first[l] = blocks;
+        a.gx[l] = (a.g[l].N + tile - 1) / tile;
+        a.gy[l] = (a.g[l].M + tile - 1) / tile;
+        blocks += a.gx[l] * a.gy[l] * gs.splits;
+    }
+    a.first[NLAYER] = blocks;
+    if (tile == 32)
+        hipLaunchKernelGGL((mlp_wgrad_all<32>), dim3((unsigned int)blocks), dim3(256), 0, h->stream, a);
+    else
+        hipLaunchKernelGGL((mlp_wgrad_all<64>), dim3((unsigned int)blocks), dim3(256), 0, h->stream, a);
+    check(hipGetLastError(), "mlp_wgrad_all launch");
 }
 
 void encode(clode_mlp *h, const float *Xdev, int n, bool train = false)
@@ -1185,19 +1475,9 @@ void download(clode_mlp *h, void *dst, const void *src, size_t bytes)
 
 void refresh_bf16(clode_mlp *h)
 {
-    std::vector<float> p(h->nparam);
-    download(h, p.data(), h->p.p, h->nparam * 4);
-    std::vector<bf16_t> b(h->nparam), bt(h->nparam, 0);
-    for (size_t i = 0; i < b.size(); ++i)
-        b[i] = f2bf(p[i]);
-    for (int l = 0; l < NLAYER; ++l) {
-        const Layer &Ly = h->L[l];
-        for (int o = 0; o < Ly.out; ++o)
-            for (int k = 0; k < Ly.in; ++k)
-                bt[Ly.woff + (size_t)k * Ly.out + o] = b[Ly.woff + (size_t)o * Ly.in + k];
-    }
-    upload(h, h->pbf.p, b.data(), b.size() * 2);
-    upload(h, h->pbfT.p, bt.data(), bt.size() * 2);
+    hipLaunchKernelGGL(mlp_put_weights, dim3((unsigned int)((h->nparam + 255) / 256)), dim3(256), 0, h->stream, h->p.p,
+                       h->copies(), h->table(), (long long)h->nparam);
+    check(hipGetLastError(), "mlp_put_weights launch");
     check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
 }
 
@@ -1265,7 +1545,7 @@ void screen_fused(clode_mlp *h, int nx, int ny, float tol, float *P, float *A, i
     a.ny = ny;
     a.Bff = h->dBff.p;
     for (int l = 0; l < NLAYER; ++l) {
-        a.W[l] = h->pbf.p + h->L[l].woff;
+        a.W[l] = h->pbfF.p + h->L[l].woff;
         a.bias[l] = h->p.p + h->L[l].boff;
         if (((uintptr_t)a.W[l] & 15) != 0)  // the kernel reads 16-byte weight fragments
             throw MlpError("screening weights are not 16-byte aligned");
@@ -1382,6 +1662,8 @@ int clode_mlp_create(clode_mlp **out, int device, unsigned long long seed)
         h->mask.alloc(h->nparam);
         h->pbf.alloc(h->nparam);
         h->pbfT.alloc(h->nparam);
+        h->pbfF.alloc(h->nparam);
+        h->pbfTF.alloc(h->nparam);
         h->wsp.alloc((size_t)KSPLIT_MAX * H * H);  // the largest weight gradient, per split
         h->wall.alloc((size_t)KSPLIT_MAX * h->nparam);  // every layer's, per split (30 MB)
         h->dBff.alloc(2 * NFF);
@@ -1547,7 +1829,6 @@ int clode_mlp_train(clode_mlp *h, const float *X, const float *T, const int *cls
     upload(h, Xall.p, X, n * 8);
     upload(h, Tall.p, T, n * 8);
     upload(h, Call.p, cls, n * 4);
-    h->ensureRows((size_t)batch);
     std::mt19937_64 rng(seed);
     // epoch e's order is a shuffle of epoch e-1's; the next epoch's shuffle
     // runs on the host while the GPU trains on the current one.  Every
@@ -1564,18 +1845,17 @@ int clode_mlp_train(clode_mlp *h, const float *X, const float *T, const int *cls
     const size_t steps_per_epoch = (n + batch - 1) / batch;
     const double total = (double)steps_per_epoch * epochs;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    LayerTable lt;
-    for (int l = 0; l < NLAYER; ++l) {
-        lt.woff[l] = (long long)h->L[l].woff;
-        lt.in[l] = h->L[l].in;
-        lt.out[l] = h->L[l].out;
-    }
-    // by default each layer's weight and input gradients share a launch and
-    // the gradient sums run inside the optimizer launch (13 launches per
-    // step); CLODE_MLP_FUSED_TRAIN=0 launches every product on its own and
-    // sums in the backward pass (22 launches, same parameters bit for bit)
+    const LayerTable lt = h->table();
+    // by default a step is three launches: the fused row-wise pass, every
+    // layer's weight-gradient products, and the optimizer with the gradient
+    // sums; CLODE_MLP_FUSED_TRAIN=0 launches every product on its own and sums
+    // in the backward pass (22 launches, same parameters bit for bit)
     const char *fa = std::getenv("CLODE_MLP_FUSED_TRAIN");
     const bool fused = !(fa && std::strcmp(fa, "0") == 0);
+    if (fused)
+        h->ensureTransposed((size_t)batch);
+    else
+        h->ensureRows((size_t)batch);
     int nbias = 0;
     for (int l = 0; l < NLAYER; ++l)
         nbias += h->L[l].out;
@@ -1588,21 +1868,44 @@ int clode_mlp_train(clode_mlp *h, const float *X, const float *T, const int *cls
         for (size_t s = 0; s < steps_per_epoch; ++s, ++step) {
             const size_t b0 = s * (size_t)batch;
             const int nb = (int)std::min<size_t>((size_t)batch, n - b0);
-            hipLaunchKernelGGL(mlp_gather, dim3((nb * NFF + 255) / 256), dim3(256), 0, h->stream, dperm.p + b0, nb,
-                               Xall.p, Tall.p, Call.p, h->T.p, h->C.p, h->ids.p, h->dBff.p, h->A0.p, h->A0t.p,
-                               ldT(nb));
-            check(hipGetLastError(), "mlp_gather launch");
-            forward(h, nb, true);
-            hipLaunchKernelGGL(mlp_loss, dim3((NHEAD * nb + 255) / 256), dim3(256), 0, h->stream, h->Zh.p, nb, h->T.p,
-                               h->C.p, h->ids.p, 1.0f / (float)nb, h->dOut.p, h->dOutT.p, ldT(nb), eloss.p + e);
-            check(hipGetLastError(), "mlp_loss launch");
             GradSources gs;
             std::memset(&gs, 0, sizeof(gs));
-            gs.part = h->wall.p;
-            gs.pstride = (long long)h->nparam;
-            gs.n = nb;
-            gs.ld = ldT(nb);
-            backward(h, nb, fused ? &gs : nullptr);
+            if (fused) {
+                FusedStep f;
+                std::memset(&f, 0, sizeof(f));
+                f.perm = dperm.p + b0;
+                f.nb = nb;
+                f.ldt = ldT(nb);
+                f.Xa = Xall.p;
+                f.Ta = Tall.p;
+                f.Ca = Call.p;
+                f.Bff = h->dBff.p;
+                for (int l = 0; l < NLAYER; ++l) {
+                    f.W[l] = h->pbfF.p + h->L[l].woff;
+                    f.WT[l] = h->pbfTF.p + h->L[l].woff;
+                    f.bias[l] = h->p.p + h->L[l].boff;
+                }
+                f.A0t = h->A0t.p;
+                for (int l = 0; l < NHID; ++l) {
+                    f.Yt[l] = h->Yt[l].p;
+                    f.dYt[l] = h->dYt[l].p;
+                }
+                f.dOutT = h->dOutT.p;
+                f.inv_n = 1.0f / (float)nb;
+                f.loss = eloss.p + e;
+                fused_step(h, f, gs);
+            } else {
+                hipLaunchKernelGGL(mlp_gather, dim3((nb * NFF + 255) / 256), dim3(256), 0, h->stream, dperm.p + b0, nb,
+                                   Xall.p, Tall.p, Call.p, h->T.p, h->C.p, h->ids.p, h->dBff.p, h->A0.p, h->A0t.p,
+                                   ldT(nb));
+                check(hipGetLastError(), "mlp_gather launch");
+                forward(h, nb, true);
+                hipLaunchKernelGGL(mlp_loss, dim3((NHEAD * nb + 255) / 256), dim3(256), 0, h->stream, h->Zh.p, nb,
+                                   h->T.p, h->C.p, h->ids.p, 1.0f / (float)nb, h->dOut.p, h->dOutT.p, ldT(nb),
+                                   eloss.p + e);
+                check(hipGetLastError(), "mlp_loss launch");
+                backward(h, nb);
+            }
             // cosine decay to 5 % of the initial rate
             const double frac = (double)step / total;
             AdamStep as;
@@ -1616,11 +1919,11 @@ int clode_mlp_train(clode_mlp *h, const float *X, const float *T, const int *cls
             const int wblocks = (int)((h->nparam + 255) / 256);
             if (fused)
                 hipLaunchKernelGGL(mlp_adam_sum, dim3((unsigned int)(wblocks + nbias)), dim3(256), 0, h->stream,
-                                   h->p.p, h->m1.p, h->m2.p, h->mask.p, h->pbf.p, h->pbfT.p, lt,
+                                   h->p.p, h->m1.p, h->m2.p, h->mask.p, h->copies(), lt,
                                    (long long)h->nparam, wblocks, gs, as);
             else
                 hipLaunchKernelGGL(mlp_adam, dim3((unsigned int)wblocks), dim3(256), 0, h->stream, h->p.p, h->g.p,
-                                   h->m1.p, h->m2.p, h->mask.p, h->pbf.p, h->pbfT.p, lt, (long long)h->nparam, as);
+                                   h->m1.p, h->m2.p, h->mask.p, h->copies(), lt, (long long)h->nparam, as);
             check(hipGetLastError(), "mlp_adam launch");
         }
         if (e + 1 < epochs) {

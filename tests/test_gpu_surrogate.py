@@ -130,8 +130,8 @@ def test_training_fits_a_smooth_map(gpu_available):
 
 @pytest.mark.parametrize("n, batch", [(16384, 1024), (5000, 2048), (3000, 64)])
 def test_fused_optimizer_matches_separate_sums(gpu_available, n, batch):
-    """The training loop's fused launches (each layer's weight and input
-    gradients in one launch, mlp_gemm_pair; the split-K sums and bias
+    """The training loop's fused launches (the row-wise pass, mlp_fused_step;
+    every layer's weight gradient, mlp_wgrad_all; the split-K sums and bias
     reductions inside the optimizer launch, mlp_adam_sum) against every
     product in a launch of its own, the backward pass's reduction launches
     and a plain Adam launch (CLODE_MLP_FUSED_TRAIN=0): same blocks, partial
@@ -153,6 +153,28 @@ def test_fused_optimizer_matches_separate_sums(gpu_available, n, batch):
     assert np.array_equal(fused.get_params(), separate.get_params())
     assert np.allclose(h_fused, h_sep, rtol=1e-5, atol=0)
     assert not np.array_equal(fused.get_params(), net(13).get_params())  # training moved the parameters
+
+
+@pytest.mark.parametrize("n, batch", [(1, 64), (17, 64), (64 + 15, 64), (129, 128), (2048 + 9, 2048), (40000, 16384)])
+def test_fused_training_pass_at_its_edges(gpu_available, n, batch):
+    """The fused training launches at the edges of their tiling: one row, a
+    partial group of 16 rows, minibatches that end one past a group or past
+    the groups of an XCD, and both sides of the weight-gradient tile rule.
+    The same blocks, K order and epilogue arithmetic as the separate launches,
+    so the parameters agree bit for bit."""
+    rng = np.random.default_rng(11)
+    U = rng.random((n, 2))
+    T, cls = smooth_targets(U)
+    out = []
+    for flag in ("1", "0"):
+        os.environ["CLODE_MLP_FUSED_TRAIN"] = flag
+        try:
+            m = net(3)
+            m.train(U, T, cls, epochs=2, batch=batch, lr=2e-3, seed=2)
+        finally:
+            del os.environ["CLODE_MLP_FUSED_TRAIN"]
+        out.append(m.get_params())
+    assert np.array_equal(out[0], out[1])
 
 
 def test_screen_flags_class_boundary(gpu_available):
