@@ -306,8 +306,10 @@ __global__ void __launch_bounds__(256) mlp_gemm(const GemmArgs g)
 __device__ __attribute__((always_inline)) inline void encode_pair(float x0, float x1, int f, const float *Bff, bf16_t &s, bf16_t &c)
 {
     const float p = 6.283185307179586f * (Bff[f] * x0 + Bff[NFF + f] * x1);
-    s = f2bf(sinf(p));
-    c = f2bf(cosf(p));
+    float sp, cp;
+    sincosf(p, &sp, &cp);  // one argument reduction for both
+    s = f2bf_dev(sp);
+    c = f2bf_dev(cp);
 }
 
 // row i of the encoded inputs; A0t (optional): transposed copy [32][ldt]
@@ -334,10 +336,11 @@ __global__ void __launch_bounds__(256) mlp_encode(const float *X, int n, const f
     encode_row(X[2 * i], X[2 * i + 1], i, Bff, A0, A0t, ldt);
 }
 
-// grid inputs: cell c = ix * ny + iy at (lo + (hi - lo) * i / (n - 1)), normalised to [0, 1]
+// grid inputs (c < nx * ny <= 2^26): cell c = ix * ny + iy at (lo + (hi - lo) * i / (n - 1)), normalised to [0, 1]
 __device__ __attribute__((always_inline)) inline void grid_point(long long c, int nx, int ny, float &x0, float &x1)
 {
-    const int ix = (int)(c / ny), iy = (int)(c % ny);
+    const unsigned int k = (unsigned int)c, n = (unsigned int)ny;
+    const int ix = (int)(k / n), iy = (int)(k - k / n * n);
     x0 = nx > 1 ? (float)ix / (float)(nx - 1) : 0.f;
     x1 = ny > 1 ? (float)iy / (float)(ny - 1) : 0.f;
 }
@@ -756,11 +759,20 @@ thread_local std::string g_err;
 // L2-resident) and the four per-cell results touch memory, where the
 // layer-by-layer path writes and re-reads 0.5 KB of activations per cell and
 // layer.  Each wave owns 64 output columns of a hidden layer (8 x 4 blocks of
-// 16 x 16) or 32 of the heads (8 x 2), takes its weight fragments straight
-// from global memory with the next K step's in flight, and reads the
-// activations from LDS.  Operand layout, K order (32-deep steps, ascending)
-// and epilogue arithmetic are those of mlp_gemm, so every output equals the
-// layer-by-layer path bit for bit.
+// 16 x 16) or 32 rows of the heads (2 x 5 blocks), takes its weight fragments
+// straight from global memory with the next K step's in flight, and reads the
+// activations from LDS.  K order (32-deep steps, ascending) and epilogue
+// arithmetic are those of mlp_gemm, so every output equals the layer-by-layer
+// path bit for bit.
+// What bounds it is the vector ALU's issue: busy 70 % of the time at 2.5 ms, the
+// matrix cores 36 %, and every instruction taken out shows (SiLU of 1024 values
+// per cell is 60 % of them).  2048 x 2048 cells: 3.45 ms with weights read row
+// by row and scalar LDS stores; 3.25 with weights in fragment order, 2.80 with
+// the weights as first operand (one 8-byte LDS store for four values), 2.5 with
+// biases in LDS and the next layer's weights on their way during the epilogue,
+// 2.30 with the prediction spread over the four waves.  Two groups of four
+// waves kept half a layer apart by shared barriers, so that one's products
+// overlap the other's epilogues, took 2.78: two workgroups that drift do better.
 //
 // LDS: the activations [SROWS][H] BF16, 64 KiB, two workgroups per CU.  The
 // 16-byte chunk kc of row m is stored at chunk kc ^ (m & 15) of that row, so
@@ -769,15 +781,15 @@ thread_local std::string g_err;
 // layer the same bytes hold the FP32 head outputs [SROWS][ZPITCH].
 constexpr int SROWS = 128;         // cells per workgroup
 constexpr int ZPITCH = NOUT + 1;   // row pitch of the head outputs (floats)
-constexpr int HBLK = (NOUT + 15) / 16;  // column blocks of the heads that hold used columns
 static_assert(SROWS * ZPITCH * 4 <= SROWS * H * 2, "head outputs fit in the activation buffer");
-static_assert(SROWS == 8 * 16 && H == 4 * 64 && NOUTP == 4 * 32, "wave tiling");
+constexpr int HBLK = (NOUT + 15) / 16;  // column blocks of the heads that hold used columns
+static_assert(SROWS == 8 * 16 && SROWS == 4 * 32 && H == 4 * 64 && NOUT % 4 == 0 && HBLK * 16 <= NOUTP, "wave tiling");
 
 struct ScreenArgs {
     long long ncell;
     int nx, ny;
     const float *Bff;
-    const bf16_t *W[NLAYER];  // Wt[out][in], BF16
+    const bf16_t *W[NLAYER];  // Wt[out][in] in fragment order
     const float *bias[NLAYER];
     const float *tm;  // tmean[2], tstd[2]
     float tol;
@@ -800,75 +812,183 @@ __device__ __attribute__((always_inline)) inline int lane_here()
 // element (m, k) of the swizzled activation tile
 __device__ __attribute__((always_inline)) inline int sw(int m, int k) { return m * H + ((((k >> 3) ^ (m & 15))) << 3) + (k & 7); }
 
-// acc[i][j] += act[rows of block i][0, K) * W[columns of block j][0, K)^T for
-// the NB column blocks starting at column n0 (16 NB columns)
+// Weight fragments in flight: K step ks of a product is in b[ks % PF], loaded
+// PF - 1 steps ahead, the first ones during the layer before.
+constexpr int PF = 2;
+
 template <int K, int NB>
-__device__ __attribute__((always_inline)) inline void screen_product(const bf16_t *act, const bf16_t *__restrict__ W, int n0, int lane,
-                                      f32x4 (&acc)[8][NB])
+__device__ __attribute__((always_inline)) inline void screen_load(const bf16_t *__restrict__ W, int n0, int ks, int lane,
+                                                                  bf16x8 (&b)[PF][NB])
+{
+    if (ks < K / TK) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            b[ks % PF][j] = *(const bf16x8 *)(W + ((n0 / 16 + j) * (K / TK) + ks) * 512 + lane * 8);
+    }
+}
+
+template <int K, int NB>
+__device__ __attribute__((always_inline)) inline void screen_first(const bf16_t *__restrict__ W, int n0, int lane,
+                                                                   bf16x8 (&b)[PF][NB])
+{
+#pragma unroll
+    for (int ks = 0; ks < PF - 1; ++ks)
+        screen_load<K, NB>(W, n0, ks, lane, b);
+}
+
+// acc[i][j] = W[columns of block j][0, K) * act[rows of block i][0, K)^T for
+// the NB column blocks starting at column n0 and the RB row blocks starting at
+// row m0.  The weights are the first MFMA operand, so a lane holds four
+// consecutive columns (lane >> 4) * 4 .. + 3 of one row lane & 15: four
+// neighbouring elements of the activation tile (the sums are those of the
+// other operand order, element by element).
+template <int K, int RB, int NB>
+__device__ __attribute__((always_inline)) inline void screen_product(const bf16_t *act, const bf16_t *__restrict__ W, int m0, int n0,
+                                      int lane, bf16x8 (&b)[PF][NB], f32x4 (&acc)[RB][NB])
 {
     constexpr int NKS = K / TK;
     const int r = lane & 15, kq = (lane >> 4) * 8;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j)
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 b[NB], bn[NB];
+    constexpr int HR = RB / 2;
+    bf16x8 a[2][HR];
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
-        b[j] = *(const bf16x8 *)(W + ((n0 / 16 + j) * NKS) * 512 + lane * 8);
-#pragma unroll 1
+    for (int i = 0; i < HR; ++i)
+        a[0][i] = *(const bf16x8 *)&act[sw(m0 + i * 16 + r, kq)];
+#pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-        if (ks + 1 < NKS) {
+        screen_load<K, NB>(W, n0, ks + PF - 1, lane, b);
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
-                bn[j] = *(const bf16x8 *)(W + ((n0 / 16 + j) * NKS + ks + 1) * 512 + lane * 8);
-        }
+        for (int h = 0; h < 2; ++h) {
+            if (h == 0 || ks + 1 < NKS) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const bf16x8 a = *(const bf16x8 *)&act[sw(i * 16 + r, ks * TK + kq)];
+                for (int i = 0; i < HR; ++i)
+                    a[1 - h][i] = *(const bf16x8 *)&act[sw(m0 + ((1 - h) * HR + i) * 16 + r, (ks + h) * TK + kq)];
+            }
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-        }
-        if (ks + 1 < NKS) {
+            for (int i = 0; i < HR; ++i)
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
-                b[j] = bn[j];
+                for (int j = 0; j < NB; ++j)
+                    acc[h * HR + i][j] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[ks % PF][j], a[h][i], acc[h * HR + i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);  // keep the loads where they are
         }
     }
 }
 
-// hidden layer in place: act <- SiLU(act W^T + bias), BF16
-template <int K>
-__device__ __attribute__((always_inline)) inline void screen_hidden(bf16_t *act, const bf16_t *__restrict__ W, const float *__restrict__ bias,
-                                     int wave, int lane)
+// hidden layer's epilogue in place: act <- SiLU(acc + bias), BF16, four elements
+// to a conversion pair and one 8-byte LDS store
+__device__ __attribute__((always_inline)) inline void screen_hidden(bf16_t *act, const f32x4 (&acc)[8][4], const float *bias, int wave)
 {
-    f32x4 acc[8][4];
-    screen_product<K, 4>(act, W, wave * 64, lane, acc);
     __syncthreads();  // every wave has read the layer's input
-    lane = lane_here();
+    const int lane = lane_here();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int n = wave * 64 + j * 16 + (lane & 15);
-        const float bj = bias[n];
+        const int n = wave * 64 + j * 16 + (lane >> 4) * 4;
+        const f32x4 bj = *(const f32x4 *)(bias + n);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float v = acc[i][j][q];
-                v += bj;
-                act[sw(i * 16 + (lane >> 4) * 4 + q, n)] = f2bf_dev(silu(v));
-            }
+        for (int i = 0; i < 8; ++i) {
+            const f32x4 v = acc[i][j] + bj;
+            const bf16x4 y = {(__bf16)silu(v[0]), (__bf16)silu(v[1]), (__bf16)silu(v[2]), (__bf16)silu(v[3])};
+            *(bf16x4 *)&act[sw(i * 16 + (lane & 15), n)] = y;
+        }
     }
     __syncthreads();
+}
+
+// One head's outputs zh in place: to feature units, and its class scores to
+// softmax values; returns its class.  The quotients by the sum are those of a
+// division: its reciprocal is refined once and every quotient corrected by its
+// remainder, three instructions instead of ten.
+__device__ __attribute__((always_inline)) inline uint8_t predict_head(float *zh, const float *tmean, const float *tstd)
+{
+    float ex[NCLS];
+#pragma unroll
+    for (int c = 0; c < NCLS; ++c)
+        ex[c] = zh[2 + c];
+    float mx = ex[0];
+    int best = 0;
+#pragma unroll
+    for (int c = 1; c < NCLS; ++c) {
+        best = ex[c] > mx ? c : best;
+        mx = ex[c] > mx ? ex[c] : mx;
+    }
+    float se = 0.f;
+#pragma unroll
+    for (int c = 0; c < NCLS; ++c) {
+        ex[c] = __expf(ex[c] - mx);
+        se += ex[c];
+    }
+    float r = __builtin_amdgcn_rcpf(se);
+    r = fmaf(fmaf(-se, r, 1.f), r, r);
+#pragma unroll
+    for (int c = 0; c < NCLS; ++c) {
+        const float q = ex[c] * r;
+        zh[2 + c] = fmaf(fmaf(-q, se, ex[c]), r, q);
+    }
+    zh[0] = expf(zh[0] * tstd[0] + tmean[0]);
+    zh[1] = zh[1] * tstd[1] + tmean[1];
+    return (uint8_t)best;
+}
+
+// The heads of one row (z, hc: what predict_head left) in two neighbouring
+// lanes: the mean period (half 0) or amplitude (half 1), and in both the class
+// and whether the heads disagree.  A half takes eight of the classes.
+__device__ __attribute__((always_inline)) inline bool predict_pair(const float *z, const uint8_t *hc, int half, float tol,
+                                                                   float &mean, int &cls)
+{
+    float v[NHEAD];
+    mean = 0.f;
+#pragma unroll
+    for (int h = 0; h < NHEAD; ++h) {
+        v[h] = z[h * HW + half];
+        mean += v[h];
+    }
+    mean *= 1.f / NHEAD;
+    bool dis = false;
+#pragma unroll
+    for (int h = 0; h < NHEAD; ++h)
+        dis |= fabsf(v[h] - mean) > tol * fabsf(mean);
+    const int c0 = half * (NCLS / 2);
+    float pbest = 0.f;
+    int best = c0;
+#pragma unroll
+    for (int c = 0; c < NCLS / 2; ++c) {
+        float p = 0.f;
+#pragma unroll
+        for (int h = 0; h < NHEAD; ++h)
+            p += z[h * HW + 2 + c0 + c];
+        if (c == 0) {
+            pbest = p;
+        } else {
+            best = p > pbest ? c0 + c : best;
+            pbest = p > pbest ? p : pbest;
+        }
+    }
+    const float po = __shfl_xor(pbest, 1);
+    const int bo = __shfl_xor(best, 1);
+    cls = half ? (pbest > po ? best : bo) : (po > pbest ? bo : best);
+#pragma unroll
+    for (int k = 0; k < NHEAD / 2; ++k)
+        dis |= hc[half * (NHEAD / 2) + k] != cls;
+    return __shfl_xor((int)dis, 1) | (int)dis;
 }
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) mlp_screen_fused(const ScreenArgs s)
 {
     __shared__ __attribute__((aligned(16))) bf16_t act[SROWS * H];
+    __shared__ __attribute__((aligned(16))) float bias[NHID * H + NOUT];
+    __shared__ uint8_t hc[SROWS * NHEAD];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const long long c0 = (long long)blockIdx.x * SROWS;
+#pragma unroll
+    for (int l = 0; l < NHID; ++l)
+        bias[l * H + t] = s.bias[l][t];
+    if (t < NOUT)
+        bias[NHID * H + t] = s.bias[NHID][t];
     {  // encode: thread t -> cell row t / 2, frequencies (t % 2) * 8 .. + 8
         const int m = t >> 1, f0 = (t & 1) * (NFF / 2);
         const long long c = c0 + m < s.ncell ? c0 + m : s.ncell - 1;
@@ -882,35 +1002,71 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
         }
     }
     __syncthreads();
-    screen_hidden<D0>(act, s.W[0], s.bias[0], wave, lane);
-    screen_hidden<H>(act, s.W[1], s.bias[1], wave, lane);
-    screen_hidden<H>(act, s.W[2], s.bias[2], wave, lane);
-    screen_hidden<H>(act, s.W[3], s.bias[3], wave, lane);
-    // heads: 128 columns, 32 per wave; the 72 used ones go to LDS in FP32
-    f32x4 acc[8][2];
-    screen_product<H, 2>(act, s.W[NHID], wave * 32, lane, acc);
+    f32x4 acc[8][4];
+    bf16x8 bw[PF][4];
+    screen_first<D0, 4>(s.W[0], wave * 64, lane, bw);
+    screen_product<D0, 8, 4>(act, s.W[0], 0, wave * 64, lane, bw, acc);
+    screen_first<H, 4>(s.W[1], wave * 64, lane, bw);
+    screen_hidden(act, acc, bias, wave);
+#pragma unroll
+    for (int l = 1; l < NHID - 1; ++l) {
+        screen_product<H, 8, 4>(act, s.W[l], 0, wave * 64, lane, bw, acc);
+        screen_first<H, 4>(s.W[l + 1], wave * 64, lane, bw);
+        screen_hidden(act, acc, bias + l * H, wave);
+    }
+    bf16x8 bh[PF][HBLK];
+    screen_product<H, 8, 4>(act, s.W[NHID - 1], 0, wave * 64, lane, bw, acc);
+    screen_first<H, HBLK>(s.W[NHID], 0, lane, bh);
+    screen_hidden(act, acc, bias + (NHID - 1) * H, wave);
+    // heads: every wave takes 32 rows and the five column blocks that hold the
+    // 72 used columns; they go to LDS in FP32
+    f32x4 az[2][HBLK];
+    screen_product<H, 2, HBLK>(act, s.W[NHID], wave * 32, 0, lane, bh, az);
     __syncthreads();  // the activations are no longer needed: z overlays them
     float *z = reinterpret_cast<float *>(act);
     const int hl = lane_here();
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = wave * 32 + j * 16 + (hl & 15);
+    for (int j = 0; j < HBLK; ++j) {
+        const int n = j * 16 + (hl >> 4) * 4;
         if (n < NOUT) {
-            const float bj = s.bias[NHID][n];
+            const f32x4 bj = *(const f32x4 *)(bias + NHID * H + n);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int i = 0; i < 2; ++i) {
+                const f32x4 v = az[i][j] + bj;
+                float *zr = z + (wave * 32 + i * 16 + (hl & 15)) * ZPITCH + n;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float v = acc[i][j][q];
-                    v += bj;
-                    z[(i * 16 + (hl >> 4) * 4 + q) * ZPITCH + n] = v;
-                }
+                for (int q = 0; q < 4; ++q)
+                    zr[q] = v[q];
+            }
         }
     }
     __syncthreads();
-    if (t < SROWS && c0 + t < s.ncell) {
-        const long long c = c0 + t;
-        predict_row(z + t * ZPITCH, s.tm, s.tm + 2, s.tol, s.period[c], s.amp[c], s.cls[c], s.flags[c]);
+    // predict_row's steps and results, over all four waves: two heads of a row
+    // to a thread, then the row's heads together in a pair of threads
+    {
+        float *zr = z + (t & 127) * ZPITCH;
+#pragma unroll
+        for (int k = 0; k < NHEAD / 2; ++k) {
+            const int h = (t >> 7) * (NHEAD / 2) + k;
+            hc[(t & 127) * NHEAD + h] = predict_head(zr + h * HW, s.tm, s.tm + 2);
+        }
+    }
+    __syncthreads();
+    {
+        const int m = t >> 1, half = t & 1;
+        const long long c = c0 + m;
+        int best;
+        float mean;
+        const bool dis = predict_pair(z + m * ZPITCH, hc + m * NHEAD, half, s.tol, mean, best);
+        if (c < s.ncell) {
+            if (half) {
+                s.amp[c] = mean;
+                s.flags[c] = dis ? 1 : 0;
+            } else {
+                s.period[c] = mean;
+                s.cls[c] = best;
+            }
+        }
     }
 }
 
@@ -918,19 +1074,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
 // One launch for everything of an optimizer step that runs row by row: gather
 // and encode, the four hidden layers, the heads, the loss, and the input
 // gradients back to the first layer.  A workgroup of 8 waves takes 16 rows of
-// the minibatch; activations and gradients stay in LDS (two 8 KiB tiles, one
-// barrier per layer), SiLU' stays in the registers of the lane that needs it
-// again (a lane forms the same elements of a layer forward and backward), and
-// each wave's weight fragments of the next product are loaded while the current
-// one runs.  Only the transposed operands of the weight-gradient products leave
-// the CU.
-// What bounds it is the chain of nine products, each waiting for the one
-// before: 17 us with 4 workgroups, 21 us with 128 (2048 rows), 23 us with 256;
-// past one workgroup per CU the weights' way from L2, 1 MB per workgroup at
-// 64 B per cycle, 17 us per 256 workgroups.  An optimizer step's three launches
-// take 40 us at 2048 rows and 29 us at 64; the thirteen that this replaces
-// (gather, five forward products, loss, five backward pairs, optimizer) took
-// 79 us and 58 us, each waiting for a few hundred workgroups to start and drain.
+// the minibatch; activations and gradients stay in LDS (8 KiB), the
+// pre-activations in the registers of the lane that needs them again (a lane
+// forms the same elements of a layer forward and backward), and each wave's
+// weight fragments of the next product are loaded while the current one runs.
+// Only the transposed operands of the weight-gradient products leave the CU.
+// What bounds it is the weights' way from L2: 1 MB per workgroup through the
+// CU's 64 B per cycle, 7 us.  The launches it replaces (gather, five forward
+// products, loss, the input gradients) took about 53 us of GPU time a step at
+// 2048 rows, each waiting for a few hundred workgroups to start and drain.
 // K order and epilogue arithmetic are those of gemm_block, so the weights
 // after training are the same bits.
 constexpr int FROWS = 16;    // rows per workgroup

@@ -223,6 +223,35 @@ def test_screen_fused_matches_layer_by_layer(gpu_available, shape):
     assert np.all(np.isfinite(fused[0])) and np.all(np.isfinite(fused[1]))
 
 
+@pytest.mark.parametrize("heads", ["all classes tie", "ties across the halves", "far apart", "infinite"])
+def test_screen_prediction_of_degenerate_heads(gpu_available, heads):
+    """The screening kernel takes a row's heads and the two halves of its
+    classes in different lanes: equal scores (the first class counts),
+    scores whose exponentials underflow, and scores that are not finite give
+    what one lane per row gives (CLODE_MLP_FUSED_SCREEN=0), bit for bit."""
+    m = net(4)
+    p = m.get_params()
+    b = p[-128:]  # the heads' biases, 18 of each: log-period, amplitude, 16 scores
+    if heads == "all classes tie":
+        p[:] = 0.0
+    elif heads == "ties across the halves":
+        p[-128 - 256 * 128:] = 0.0
+        b[[2 + 3, 2 + 12, 20 + 12, 38 + 3, 56 + 12]] = 2.0
+    elif heads == "far apart":
+        b[2:72] = np.linspace(-400.0, 400.0, 70)
+    else:
+        b[[2 + 9, 20 + 1]] = np.inf, -np.inf
+    m.set_params(p)
+    fused = m.screen_grid(37, 11, tol=0.05, dilate=0)
+    os.environ["CLODE_MLP_FUSED_SCREEN"] = "0"
+    try:
+        layered = m.screen_grid(37, 11, tol=0.05, dilate=0)
+    finally:
+        del os.environ["CLODE_MLP_FUSED_SCREEN"]
+    for a, b in zip(fused, layered):
+        assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
+
+
 def lactotroph_solver(n_axis_check=None):
     import clode_amd as clode
     from clode_amd.surrogate import integrator_solver
