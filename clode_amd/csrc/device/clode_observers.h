@@ -93,8 +93,8 @@ CLODE_DEV void runningMean(obsreal &mean, obsreal newValue, unsigned int eventCo
 }
 
 // extrema (fp32c programs run in the non-IEEE mode, where fmax and fmin are
-// single instructions already)
-#if CLODE_PREC == 3
+// single instructions already; a host compile has no instructions to choose)
+#if CLODE_PREC == 3 || !defined(__AMDGCN__)
 template <class T>
 CLODE_DEV T obs_max(T a, T b) { return fmax(a, b); }
 template <class T>
