@@ -671,27 +671,53 @@ extern "C" __global__ void __launch_bounds__(CLODE_BLOCK_MAX) CLODE_KERNEL_ATTRS
     run_member<FeaturesLane>(s.fe, sp, i);
 }
 
-// The feature matrix F ([nF][nPts], member index fastest, as the observers
-// write it) as double, member-major ([nPts][nF]): the layout the host API
-// hands out, transposed here instead of on the host.  A block moves a tile
-// of 64 members x 32 features through LDS, so that both the reads (along
-// members) and the writes (along features) are contiguous runs.
-extern "C" __global__ void __launch_bounds__(64) clode_f_members(const ostore *F, double *out, unsigned int nPts,
-                                                                unsigned int nF)
+#endif  // CLODE_OBSERVER
+
+// Rows of member values ([nRows][stride], member index fastest: the feature
+// matrix, the stored trajectories) as double, member-major ([count][nRows],
+// members first .. first + count - 1): the layout the host API hands out,
+// transposed here instead of on the host.  A block moves tiles of 64 members
+// x 32 rows through LDS, so that both the reads (along members) and the writes
+// (along rows) are contiguous runs; tiles are dealt out over the grid, rows
+// fastest, so that the lines of a member's output that two tiles share are
+// written close together.
+template <class T>
+CLODE_DEV void members_tiles(const T *src, double *out, unsigned int stride, unsigned int first, unsigned int count,
+                             unsigned long long nRows, double (*tile)[65])
 {
-    __shared__ double tile[32][65];
-    const unsigned int m0 = blockIdx.x * 64u, f0 = blockIdx.y * 32u, t = threadIdx.x;
-    for (unsigned int k = 0; k < 32u; ++k)
-        if (f0 + k < nF && m0 + t < nPts)
-            tile[k][t] = (double)F[(size_t)(f0 + k) * nPts + m0 + t];
-    __syncthreads();
-    for (unsigned int L = t; L < 64u * 32u; L += 64u) {
-        const unsigned int r = L / 32u, c = L % 32u;
-        if (m0 + r < nPts && f0 + c < nF)
-            out[(size_t)(m0 + r) * nF + f0 + c] = tile[c][r];
+    const unsigned int t = threadIdx.x;
+    const unsigned long long rowTiles = (nRows + 31) / 32, tiles = ((unsigned long long)count + 63) / 64 * rowTiles;
+    for (unsigned long long k = blockIdx.x; k < tiles; k += gridDim.x) {
+        const unsigned long long r0 = k % rowTiles * 32;
+        const unsigned int m0 = (unsigned int)(k / rowTiles * 64);
+        for (unsigned int r = 0; r < 32u; ++r)
+            if (r0 + r < nRows && m0 + t < count)
+                tile[r][t] = (double)src[(size_t)(r0 + r) * stride + first + m0 + t];
+        __syncthreads();
+        for (unsigned int L = t; L < 64u * 32u; L += 64u) {
+            const unsigned int m = L / 32u, r = L % 32u;
+            if (m0 + m < count && r0 + r < nRows)
+                out[(size_t)(m0 + m) * nRows + r0 + r] = tile[r][m];
+        }
+        __syncthreads();
     }
 }
-#endif  // CLODE_OBSERVER
+
+extern "C" __global__ void __launch_bounds__(64)
+    clode_members_f64(const double *src, double *out, unsigned int stride, unsigned int first, unsigned int count,
+                      unsigned long long nRows)
+{
+    __shared__ double tile[32][65];
+    members_tiles(src, out, stride, first, count, nRows, tile);
+}
+
+extern "C" __global__ void __launch_bounds__(64)
+    clode_members_f32(const float *src, double *out, unsigned int stride, unsigned int first, unsigned int count,
+                      unsigned long long nRows)
+{
+    __shared__ double tile[32][65];
+    members_tiles(src, out, stride, first, count, nRows, tile);
+}
 #endif  // CLODE_BATCH
 
 #endif  // CLODE_KERNELS_H

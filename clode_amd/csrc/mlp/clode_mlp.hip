@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "../../../include/clode_mlp.h"
+#include "../runtime/staged_copy.h"
 
 // Staging memory of clode_mlp_screen_grid_noalloc: one byte per grid cell for
 // the dilation's second flag buffer.  Each device holds its own copy of the
@@ -1386,6 +1387,11 @@ struct clode_mlp {
     double lastMs = 0;
     size_t rows = 0;
     unsigned char *stage = nullptr;  // this device's static scratch (no-allocation screening)
+    // outputs of the last screening, kept for the next up to GRID_KEEP cells
+    Dev<float> gP, gA;
+    Dev<int> gC;
+    Dev<uint8_t> gF, gF2;
+    std::shared_ptr<clode::StagedCopy> staging;
 
     WeightCopies copies() const { return {pbf.p, pbfT.p, pbfF.p, pbfTF.p}; }
     LayerTable table() const
@@ -1480,6 +1486,7 @@ GemmArgs ga() { GemmArgs a; std::memset(&a, 0, sizeof(a)); return a; }
 
 inline int ldT(int n) { return (n + FROWS - 1) / FROWS * FROWS; }
 
+constexpr long long GRID_KEEP = 1ll << 23;  // screening outputs kept between calls: 14 bytes per cell, 117 MB
 constexpr int KSPLIT_MAX = 32;    // partial products per weight gradient
 constexpr int KSPLIT_ROWS = 256;  // rows per partial product (at least)
 
@@ -1621,8 +1628,9 @@ void upload(clode_mlp *h, void *dst, const void *src, size_t bytes)
 }
 void download(clode_mlp *h, void *dst, const void *src, size_t bytes)
 {
-    check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream), "hipMemcpy D2H");
-    check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+    if (!h->staging)
+        h->staging = clode::StagedCopy::get();
+    check(h->staging->toHost(h->device, dst, src, bytes, h->stream), "hipMemcpy D2H");
 }
 
 void refresh_bf16(clode_mlp *h)
@@ -1647,6 +1655,45 @@ float loss_grad(clode_mlp *h, int n)
     download(h, &l, h->loss.p, 4);
     return l;
 }
+
+// Standard normal deviates by the polar method (Marsaglia and Bray 1964), two
+// from each accepted point of the unit disc, the second coordinate's first.  The
+// values are those that std::normal_distribution<float> gives here; that one
+// works out the generator's range in long double for every draw, 30 ns of them,
+// and a network's 230,000 initial weights took 7 of the 9 ms of its creation.
+class Normals {
+    std::mt19937_64 rng;
+    float kept = 0.f;
+    bool have = false;
+    float uniform()  // [0, 1)
+    {
+        // through a signed conversion, the lost bit kept as a sticky one: the
+        // unsigned conversion branches on a random bit
+        const uint64_t w = rng();
+        const float u = w >> 32 ? (float)(int64_t)(w >> 1 | (w & 1)) * 0x1p-63f : (float)(int64_t)w * 0x1p-64f;
+        return u < 1.f ? u : 0x1.fffffep-1f;
+    }
+
+public:
+    explicit Normals(unsigned long long seed) : rng(seed) {}
+    float operator()()
+    {
+        if (have) {
+            have = false;
+            return kept;
+        }
+        float x, y, r2;
+        do {
+            x = 2.f * uniform() - 1.f;
+            y = 2.f * uniform() - 1.f;
+            r2 = x * x + y * y;
+        } while (r2 > 1.f || r2 == 0.f);
+        const float scale = std::sqrt(-2.f * std::log(r2) / r2);
+        kept = x * scale;
+        have = true;
+        return y * scale;
+    }
+};
 
 // a caller's pointer that must not be null
 template <class T>
@@ -1784,8 +1831,7 @@ int clode_mlp_create(clode_mlp **out, int device, unsigned long long seed)
         }
         h->nparam = off;
         // He-style initialisation for SiLU layers, small heads; Fourier frequencies ~ N(0, 3^2)
-        std::mt19937_64 rng(seed);
-        std::normal_distribution<float> nd01(0.f, 1.f);
+        Normals nd01(seed);
         std::vector<float> p(h->nparam, 0.f);
         std::vector<uint8_t> mask(h->nparam, 1);
         for (int l = 0; l < NLAYER; ++l) {
@@ -1798,7 +1844,7 @@ int clode_mlp_create(clode_mlp **out, int device, unsigned long long seed)
                         mask[k] = 0;  // padding columns stay zero
                         continue;
                     }
-                    p[k] = sd * nd01(rng);
+                    p[k] = sd * nd01();
                 }
             if (l == NHID)
                 for (int o = NOUT; o < NOUTP; ++o)
@@ -1806,7 +1852,7 @@ int clode_mlp_create(clode_mlp **out, int device, unsigned long long seed)
         }
         h->Bff.resize(2 * NFF);
         for (auto &b : h->Bff)
-            b = 3.f * nd01(rng);
+            b = 3.f * nd01();
         h->p.alloc(h->nparam);
         h->g.alloc(h->nparam);
         h->m1.alloc(h->nparam);
@@ -2122,9 +2168,9 @@ int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, f
     const int chunk = (int)std::min<long long>(ncell, 1 << 18);
     if (!fused)
         h->ensureRows((size_t)chunk);
-    Dev<float> dP, dA;
-    Dev<int> dC;
-    Dev<uint8_t> dF, dF2;
+    Dev<float> &dP = h->gP, &dA = h->gA;
+    Dev<int> &dC = h->gC;
+    Dev<uint8_t> &dF = h->gF, &dF2 = h->gF2;
     dP.alloc(ncell);
     dA.alloc(ncell);
     dC.alloc(ncell);
@@ -2153,6 +2199,13 @@ int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, f
     float ms = 0;
     (void)hipEventElapsedTime(&ms, h->ev0, h->ev1);
     h->lastMs = ms;
+    if (ncell > GRID_KEEP) {  // a grid this large is given back at once
+        dP.free();
+        dA.free();
+        dC.free();
+        dF.free();
+        dF2.free();
+    }
     MLP_CATCH
 }
 

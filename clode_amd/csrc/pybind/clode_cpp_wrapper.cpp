@@ -549,6 +549,23 @@ public:
         check(clode_get_aux(sim_, v.mutable_data(), (size_t)v.size()));
         return v;
     }
+    // member-major: shape (members, samples) for t, (members, samples, k) else
+    DArray members(int (*get)(clode_sim *, double *, size_t), py::ssize_t k)
+    {
+        size_t nt, nx, na;
+        sizes(nt, nx, na);
+        const py::ssize_t n = (py::ssize_t)n_pts(), store = n > 0 ? (py::ssize_t)nt / n : 0;
+        DArray v = k < 0 ? DArray({n, store}) : DArray({n, store, k});
+        {
+            py::gil_scoped_release nogil;
+            check(get(sim_, v.mutable_data(), (size_t)v.size()));
+        }
+        return v;
+    }
+    DArray get_t_members() { return members(clode_get_t_members, -1); }
+    DArray get_x_members() { return members(clode_get_x_members, pi_.num_var); }
+    DArray get_dx_members() { return members(clode_get_dx_members, pi_.num_var); }
+    DArray get_aux_members() { return members(clode_get_aux_members, pi_.num_aux); }
     std::vector<int> get_n_stored()
     {
         std::vector<int> v((size_t)n_pts());
@@ -901,6 +918,10 @@ PYBIND11_MODULE(clode_cpp_wrapper, m)
         .def("get_x", &TrajectorySimulatorBasePy::get_x)
         .def("get_dx", &TrajectorySimulatorBasePy::get_dx)
         .def("get_aux", &TrajectorySimulatorBasePy::get_aux)
+        .def("get_t_members", &TrajectorySimulatorBasePy::get_t_members)
+        .def("get_x_members", &TrajectorySimulatorBasePy::get_x_members)
+        .def("get_dx_members", &TrajectorySimulatorBasePy::get_dx_members)
+        .def("get_aux_members", &TrajectorySimulatorBasePy::get_aux_members)
         .def("get_n_stored", &TrajectorySimulatorBasePy::get_n_stored);
 
     m.def(

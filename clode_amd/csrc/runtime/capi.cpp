@@ -68,6 +68,12 @@ static T *need(T *p, const char *what)
 }
 
 // a caller's input array of n elements (null only when n == 0)
+static const double *in_array(const double *p, size_t n, const char *what)
+{
+    if (!p && n > 0)
+        throw InvalidArgument(std::string("null ") + what);
+    return p;
+}
 static std::vector<double> in_vec(const double *p, size_t n, const char *what)
 {
     if (!p && n > 0)
@@ -150,6 +156,14 @@ static std::string join(const std::vector<std::string> &v)
         s += v[i];
     }
     return s;
+}
+
+// a caller's output array of n elements (null only when n == 0)
+static double *out_array(double *p, size_t n)
+{
+    if (!p && n > 0)
+        throw InvalidArgument("null output buffer");
+    return p;
 }
 
 static int copy_vec(const std::vector<double> &v, double *out, size_t n)
@@ -259,7 +273,7 @@ int clode_compile(clode_sim *sim)
 int clode_set_problem_data(clode_sim *sim, const double *x0, size_t nx0, const double *pars, size_t npars)
 {
     CHECK_SIM(sim) CLODE_TRY
-    sim->s->setProblemData(in_vec(x0, nx0, "x0"), in_vec(pars, npars, "pars"));
+    sim->s->setProblemData(in_array(x0, nx0, "x0"), nx0, in_array(pars, npars, "pars"), npars);
     CLODE_CATCH
 }
 int clode_set_tspan(clode_sim *sim, const double *tspan, size_t n)
@@ -269,12 +283,12 @@ int clode_set_tspan(clode_sim *sim, const double *tspan, size_t n)
 }
 int clode_set_x0(clode_sim *sim, const double *x0, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY sim->s->setX0(in_vec(x0, n, "x0"));
+    CHECK_SIM(sim) CLODE_TRY sim->s->setX0(in_array(x0, n, "x0"), n);
     CLODE_CATCH
 }
 int clode_set_pars(clode_sim *sim, const double *pars, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY sim->s->setPars(in_vec(pars, n, "pars"));
+    CHECK_SIM(sim) CLODE_TRY sim->s->setPars(in_array(pars, n, "pars"), n);
     CLODE_CATCH
 }
 int clode_set_solver_params(clode_sim *sim, const clode_solver_params *sp)
@@ -352,22 +366,22 @@ int clode_get_pars(clode_sim *sim, double *out, size_t n)
 }
 int clode_get_x0(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getX0(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getX0(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_xf(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getXf(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getXf(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_dt(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getDt(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getDt(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_tf(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getTf(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getTf(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_available_steppers(clode_sim *sim, char *buf, size_t cap, size_t *needed)
@@ -528,22 +542,42 @@ int clode_get_trajectory_sizes(clode_sim *sim, size_t *nt, size_t *nx, size_t *n
 }
 int clode_get_t(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getT(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getT(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_x(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getX(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getX(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_dx(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getDx(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getDx(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_aux(clode_sim *sim, double *out, size_t n)
 {
-    CHECK_SIM(sim) CLODE_TRY return copy_vec(sim->s->getAux(), out, n);
+    CHECK_SIM(sim) CLODE_TRY sim->s->getAux(out_array(out, n), n);
+    CLODE_CATCH
+}
+int clode_get_t_members(clode_sim *sim, double *out, size_t n)
+{
+    CHECK_SIM(sim) CLODE_TRY sim->s->getTMembers(out_array(out, n), n);
+    CLODE_CATCH
+}
+int clode_get_x_members(clode_sim *sim, double *out, size_t n)
+{
+    CHECK_SIM(sim) CLODE_TRY sim->s->getXMembers(out_array(out, n), n);
+    CLODE_CATCH
+}
+int clode_get_dx_members(clode_sim *sim, double *out, size_t n)
+{
+    CHECK_SIM(sim) CLODE_TRY sim->s->getDxMembers(out_array(out, n), n);
+    CLODE_CATCH
+}
+int clode_get_aux_members(clode_sim *sim, double *out, size_t n)
+{
+    CHECK_SIM(sim) CLODE_TRY sim->s->getAuxMembers(out_array(out, n), n);
     CLODE_CATCH
 }
 int clode_get_n_stored(clode_sim *sim, int *out, size_t n)

@@ -61,6 +61,7 @@ Simulator::~Simulator()
 void Simulator::setProblemInfo(const ProblemInfo &pi)
 {
     ++inputGen;
+    ++configGen;
     if (pi.nVar <= 0)
         throw InvalidArgument("the problem must have at least one state variable");
     if (pi.nPar < 0 || pi.nAux < 0 || pi.nWiener < 0)
@@ -75,6 +76,7 @@ void Simulator::setProblemInfo(const ProblemInfo &pi)
 void Simulator::setStepper(const std::string &s)
 {
     ++inputGen;
+    ++configGen;
     if (stepper_map().find(s) != stepper_map().end())
         stepper = s;
     else
@@ -86,6 +88,7 @@ void Simulator::setStepper(const std::string &s)
 void Simulator::setPrecision(int p)
 {
     ++inputGen;
+    ++configGen;
     if (p < PREC_SINGLE || p > PREC_FP32C)
         throw InvalidArgument("precision must be 1 (single), 2 (double) or 3 (fp32c)");
     if (p != prec) {
@@ -147,25 +150,22 @@ ProgramConfig Simulator::programConfig() const
 
 std::shared_ptr<Program> Simulator::currentProgram()
 {
-    ProgramConfig c = programConfig();
-    std::string key = compose_source(c);
-    if (!program || key != programKeyCache) {
-        program = get_program(c, root.empty() ? std::string() : root);
-        programKeyCache = key;
+    if (!program || programGen != configGen) {
+        program = get_program(programConfig(), root);
+        programGen = configGen;
     }
     return program;
 }
 
 std::shared_ptr<Program> Simulator::variantProgram(int waves, bool replay)
 {
-    ProgramConfig c = programConfig();
-    c.wavesPerEU = waves;
-    c.replay = replay;
-    std::string key = compose_source(c);
     auto &slot = programsW[2 * waves + (replay ? 1 : 0)];
-    if (!slot.second || key != slot.first) {
-        slot.second = get_program(c, root.empty() ? std::string() : root);
-        slot.first = key;
+    if (!slot.second || slot.first != configGen) {
+        ProgramConfig c = programConfig();
+        c.wavesPerEU = waves;
+        c.replay = replay;
+        slot.second = get_program(c, root);
+        slot.first = configGen;
     }
     return slot.second;
 }
@@ -245,42 +245,37 @@ void Simulator::ensureStream()
     }
 }
 
-void Simulator::upload(DeviceBuffer &b, const std::vector<double> &v, size_t elem)
+void Simulator::upload(DeviceBuffer &b, const double *v, size_t n, size_t elem)
 {
     ensureStream();
-    if (v.empty())
+    if (n == 0)
         return;
-    if (elem == 8) {
-        hip_check(hipMemcpyAsync(b.ptr, v.data(), v.size() * 8, hipMemcpyHostToDevice, stream), "hipMemcpy H2D");
-    } else {
-        std::vector<float> f(v.begin(), v.end());
-        hip_check(hipMemcpyAsync(b.ptr, f.data(), f.size() * 4, hipMemcpyHostToDevice, stream), "hipMemcpy H2D");
-        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-        return;
+    std::vector<float> f;
+    const void *src = v;
+    if (elem != 8) {
+        f.assign(v, v + n);
+        src = f.data();
     }
+    hip_check(hipMemcpyAsync(b.ptr, src, n * elem, hipMemcpyHostToDevice, stream), "hipMemcpy H2D");
     hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
 }
 
-std::vector<double> Simulator::download(const DeviceBuffer &b, size_t n, size_t elem)
+void Simulator::toHost(void *dst, const void *src, size_t bytes)
 {
-    ensureStream();
-    std::vector<double> out(n);
-    if (n == 0 || !b.ptr)
-        return out;
-    if (elem == 8) {
-        hip_check(hipMemcpyAsync(out.data(), b.ptr, n * 8, hipMemcpyDeviceToHost, stream), "hipMemcpy D2H");
-        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    } else {
-        std::vector<float> f(n);
-        hip_check(hipMemcpyAsync(f.data(), b.ptr, n * 4, hipMemcpyDeviceToHost, stream), "hipMemcpy D2H");
-        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-        std::copy(f.begin(), f.end(), out.begin());
-    }
-    return out;
+    if (!staging)
+        staging = StagedCopy::get();
+    hip_check(staging->toHost(device, dst, src, bytes, stream), "hipMemcpy D2H");
 }
 
-void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, double *out)
+static void require_capacity(size_t cap, size_t n)
 {
+    if (cap < n)
+        throw InvalidArgument("output buffer too small: need " + std::to_string(n));
+}
+
+void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, double *out, size_t cap)
+{
+    require_capacity(cap, n);
     ensureStream();
     if (n == 0)
         return;
@@ -289,13 +284,50 @@ void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, doubl
         return;
     }
     if (elem == 8) {
-        hip_check(hipMemcpyAsync(out, b.ptr, n * 8, hipMemcpyDeviceToHost, stream), "hipMemcpy D2H");
-        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        toHost(out, b.ptr, n * 8);
     } else {
         std::vector<float> f(n);
-        hip_check(hipMemcpyAsync(f.data(), b.ptr, n * 4, hipMemcpyDeviceToHost, stream), "hipMemcpy D2H");
-        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        toHost(f.data(), b.ptr, n * 4);
         std::copy(f.begin(), f.end(), out);
+    }
+}
+
+// The transposition runs on the device (clode_members_*), a block of members
+// at a time so that the copy takes at most 256 MiB beside the data (one
+// member's rows where those are more).
+void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out, size_t cap)
+{
+    const size_t n = nPts > 0 ? (size_t)nPts : 0;
+    require_capacity(cap, n * rows);
+    if (n * rows == 0)
+        return;
+    if (!b.ptr) {
+        std::fill(out, out + n * rows, 0.0);
+        return;
+    }
+    ensureStream();
+    size_t block = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (rows * 8)));
+    while (!d_members.ptr || d_members.device != device || d_members.bytes < block * rows * 8) {
+        try {
+            d_members.allocate(device, block * rows * 8);
+        } catch (const std::exception &) {  // a nearly full device: smaller blocks
+            (void)hipGetLastError();
+            if (block == 1)
+                throw;
+            block /= 2;
+        }
+    }
+    hipFunction_t fn = currentProgram()->function(device, elem == 8 ? "clode_members_f64" : "clode_members_f32");
+    for (size_t m0 = 0; m0 < n; m0 += block) {
+        const void *src = b.ptr;
+        void *dst = d_members.ptr;
+        unsigned int stride = (unsigned int)n, first = (unsigned int)m0, count = (unsigned int)std::min(block, n - m0);
+        unsigned long long nr = rows;
+        void *params[] = {&src, &dst, &stride, &first, &count, &nr};
+        const unsigned long long tiles = ((unsigned long long)count + 63) / 64 * ((nr + 31) / 32);
+        const unsigned int grid = (unsigned int)std::min<unsigned long long>(tiles, 1u << 20);
+        hip_check(hipModuleLaunchKernel(fn, grid, 1, 1, 64, 1, 1, 0, stream, params, nullptr), "launch clode_members");
+        toHost(out + m0 * rows, d_members.ptr, (size_t)count * rows * 8);
     }
 }
 
@@ -314,17 +346,17 @@ void Simulator::setNpts(int newNpts)
     if (total && largest > total)
         throw InvalidArgument("nPts*nVar, nPts*nPar, or nPts*nAux is too large");
     nPts = newNpts;
-    x0.assign((size_t)prob.nVar * nPts, 0.0);
+    const size_t nx = (size_t)prob.nVar * nPts;
     pars.assign((size_t)prob.nPar * nPts, 0.0);
     rngHost.assign(2 * (size_t)nPts, 0);
     dtHost.assign(nPts, sp.dt);
-    d_x0.allocate(device, x0.size() * wideSize());
+    d_x0.allocate(device, nx * wideSize());
     d_pars.allocate(device, pars.size() * realSize());
     d_rng.allocate(device, rngHost.size() * 8);
     d_dt.allocate(device, (size_t)nPts * wideSize());
     d_tf.allocate(device, (size_t)nPts * wideSize());
-    d_xf.allocate(device, x0.size() * wideSize());
-    upload(d_dt, dtHost, wideSize());
+    d_xf.allocate(device, nx * wideSize());
+    upload(d_dt, dtHost.data(), dtHost.size(), wideSize());
     memberTspan = false;
     d_tspan_m.release();
     d_qorder.release();
@@ -334,53 +366,52 @@ void Simulator::setNpts(int newNpts)
 }
 
 // CLODE::setProblemData (CLODE.cpp:245-280)
-void Simulator::setProblemData(const std::vector<double> &nx0, const std::vector<double> &npars)
+void Simulator::setProblemData(const double *nx0, size_t sx0, const double *npars, size_t spars)
 {
     ++inputGen;
-    if (nx0.size() % prob.nVar != 0) {
+    if (sx0 % prob.nVar != 0) {
         log_msg(LOG_INFO, "Invalid initial condition vector: not a multiple of nVar=" + std::to_string(prob.nVar));
         log_msg(LOG_INFO, "...Initial conditions were not updated!");
         return;
     }
-    if (prob.nPar > 0 && npars.size() % prob.nPar != 0) {
+    if (prob.nPar > 0 && spars % prob.nPar != 0) {
         log_msg(LOG_INFO, "Invalid parameter vector: not a multiple of nPar=" + std::to_string(prob.nPar));
         log_msg(LOG_INFO, "...Parameters were not updated!");
         return;
     }
-    int nx = (int)(nx0.size() / prob.nVar);
-    int np = prob.nPar > 0 ? (int)(npars.size() / prob.nPar) : nx;
+    int nx = (int)(sx0 / prob.nVar);
+    int np = prob.nPar > 0 ? (int)(spars / prob.nPar) : nx;
     if (nx != np) {
         log_msg(LOG_INFO, "Initial contition and parameter vector dimensions don't match");
         log_msg(LOG_INFO, "...Problem data was not updated!");
         return;
     }
     setNpts(nx);
-    setX0(nx0);
-    setPars(npars);
+    setX0(nx0, sx0);
+    setPars(npars, spars);
 }
 
 // CLODE::setX0 (CLODE.cpp:283-315)
-void Simulator::setX0(const std::vector<double> &nx0)
+void Simulator::setX0(const double *nx0, size_t n)
 {
     ++inputGen;
-    if (nPts > 0 && nx0.size() == (size_t)nPts * prob.nVar) {
-        x0 = nx0;
-        upload(d_x0, x0, wideSize());
+    if (nPts > 0 && n == (size_t)nPts * prob.nVar) {
+        upload(d_x0, nx0, n, wideSize());
     } else {
         log_msg(LOG_INFO, "...Initial conditions were not updated!");
     }
 }
 
 // CLODE::setPars (CLODE.cpp:318-350)
-void Simulator::setPars(const std::vector<double> &np)
+void Simulator::setPars(const double *np, size_t n)
 {
     ++inputGen;
-    if (nPts > 0 && np.size() == (size_t)nPts * prob.nPar) {
-        pars = np;
-        upload(d_pars, pars, realSize());
+    if (nPts > 0 && n == (size_t)nPts * prob.nPar) {
+        pars.assign(np, np + n);
+        upload(d_pars, np, n, realSize());
     } else {
         log_msg(LOG_INFO, "Invalid parameter vector: Expected " + std::to_string(nPts) + "*" +
-                              std::to_string(prob.nPar) + " elements, received " + std::to_string(np.size()));
+                              std::to_string(prob.nPar) + " elements, received " + std::to_string(n));
         log_msg(LOG_INFO, "...Parameters were not updated!");
     }
 }
@@ -404,7 +435,7 @@ void Simulator::setSolverParams(const SolverParams &nsp)
     sp = nsp;
     std::fill(dtHost.begin(), dtHost.end(), sp.dt);
     if (dtRefresh && nPts > 0)
-        upload(d_dt, dtHost, wideSize());
+        upload(d_dt, dtHost.data(), dtHost.size(), wideSize());
 }
 
 // CLODE::seedRNG() (CLODE.cpp:420-444)
@@ -660,31 +691,10 @@ void Simulator::shiftX0()
 }
 
 // CLODE::getX0 / getXf / getDt / getTf (CLODE.cpp:517-583)
-std::vector<double> Simulator::getX0()
-{
-    if (nPts <= 0)
-        return {};
-    x0 = download(d_x0, (size_t)prob.nVar * nPts, wideSize());
-    return x0;
-}
-std::vector<double> Simulator::getXf()
-{
-    if (nPts <= 0)
-        return {};
-    return download(d_xf, (size_t)prob.nVar * nPts, wideSize());
-}
-std::vector<double> Simulator::getDt()
-{
-    if (nPts <= 0)
-        return {};
-    return download(d_dt, (size_t)nPts, wideSize());
-}
-std::vector<double> Simulator::getTf()
-{
-    if (nPts <= 0)
-        return {};
-    return download(d_tf, (size_t)nPts, wideSize());
-}
+void Simulator::getX0(double *out, size_t cap) { downloadInto(d_x0, nPts > 0 ? (size_t)prob.nVar * nPts : 0, wideSize(), out, cap); }
+void Simulator::getXf(double *out, size_t cap) { downloadInto(d_xf, nPts > 0 ? (size_t)prob.nVar * nPts : 0, wideSize(), out, cap); }
+void Simulator::getDt(double *out, size_t cap) { downloadInto(d_dt, nPts > 0 ? (size_t)nPts : 0, wideSize(), out, cap); }
+void Simulator::getTf(double *out, size_t cap) { downloadInto(d_tf, nPts > 0 ? (size_t)nPts : 0, wideSize(), out, cap); }
 
 // ------------------------------------------------------------------ features
 
@@ -701,6 +711,7 @@ void Simulator::updateObserverInfo()
 void Simulator::setObserverParams(const ObserverParams &nop)
 {
     ++inputGen;
+    ++configGen;
     if (nop.eVarIx >= (unsigned int)prob.nVar || nop.fVarIx >= (unsigned int)prob.nVar)
         throw InvalidArgument("observer eVarIx/fVarIx must index a state variable");
     op = nop;
@@ -711,6 +722,7 @@ void Simulator::setObserverParams(const ObserverParams &nop)
 void Simulator::setObserver(const std::string &name)
 {
     ++inputGen;
+    ++configGen;
     if (observer_map().find(name) != observer_map().end()) {
         observer = name;
         updateObserverInfo();
@@ -865,45 +877,26 @@ void Simulator::transientFeatures(double tr0, double tr1, double fe0, double fe1
 }
 
 // CLODEfeatures::getF (CLODEfeatures.cpp:261-275)
-std::vector<double> Simulator::getF()
-{
-    if (nPts <= 0 || !d_F.ptr)
-        return std::vector<double>(Felements, 0.0);
-    return download(d_F, Felements, wideSize());
-}
-
 void Simulator::getFInto(double *out, size_t cap)
 {
-    if (cap < Felements)
-        throw InvalidArgument("output buffer too small: need " + std::to_string(Felements));
+    require_capacity(cap, Felements);
     if (nPts <= 0 || !d_F.ptr) {
         std::fill(out, out + Felements, 0.0);
         return;
     }
-    downloadInto(d_F, Felements, wideSize(), out);
+    downloadInto(d_F, Felements, wideSize(), out, cap);
 }
 
 // The Python API's layout, F[member][feature] (features.py:467-507 reshapes
 // the reference's feature-major vector to it on the host).
 void Simulator::getFMembers(double *out, size_t cap)
 {
-    if (cap < Felements)
-        throw InvalidArgument("output buffer too small: need " + std::to_string(Felements));
+    require_capacity(cap, Felements);
     if (nPts <= 0 || !d_F.ptr || Felements == 0) {
         std::fill(out, out + Felements, 0.0);
         return;
     }
-    ensureStream();
-    if (!d_Fm.ptr || d_Fm.bytes != Felements * 8)
-        d_Fm.allocate(device, Felements * 8);
-    hipFunction_t fn = currentProgram()->function(device, "clode_f_members");
-    const void *src = d_F.ptr;
-    void *dst = d_Fm.ptr;
-    unsigned int n = (unsigned int)nPts, nF = (unsigned int)(Felements / (size_t)nPts);
-    void *params[] = {&src, &dst, &n, &nF};
-    hip_check(hipModuleLaunchKernel(fn, (n + 63u) / 64u, (nF + 31u) / 32u, 1, 64, 1, 1, 0, stream, params, nullptr),
-              "launch clode_f_members");
-    downloadInto(d_Fm, Felements, 8, out);
+    downloadMembers(d_F, Felements / (size_t)nPts, wideSize(), out, cap);
 }
 
 // ---------------------------------------------------------------- trajectory
@@ -942,10 +935,35 @@ void Simulator::trajectory()
 }
 
 // CLODEtrajectory::getT / getX / getDx / getAux / getNstored (CLODEtrajectory.cpp:132-205)
-std::vector<double> Simulator::getT() { return download(d_t, telements, wideSize()); }
-std::vector<double> Simulator::getX() { return download(d_x, xelements, realSize()); }
-std::vector<double> Simulator::getDx() { return download(d_dx, xelements, realSize()); }
-std::vector<double> Simulator::getAux() { return download(d_aux, auxelements, realSize()); }
+void Simulator::getT(double *out, size_t cap) { downloadInto(d_t, telements, wideSize(), out, cap); }
+void Simulator::getX(double *out, size_t cap) { downloadInto(d_x, xelements, realSize(), out, cap); }
+void Simulator::getDx(double *out, size_t cap) { downloadInto(d_dx, xelements, realSize(), out, cap); }
+void Simulator::getAux(double *out, size_t cap) { downloadInto(d_aux, auxelements, realSize(), out, cap); }
+void Simulator::requireTrajectories() const
+{
+    if (telements != (size_t)nStoreMax * (size_t)(nPts > 0 ? nPts : 0))
+        throw InvalidArgument("the stored trajectories are those of another ensemble size");
+}
+void Simulator::getTMembers(double *out, size_t cap)
+{
+    requireTrajectories();
+    downloadMembers(d_t, nStoreMax, wideSize(), out, cap);
+}
+void Simulator::getXMembers(double *out, size_t cap)
+{
+    requireTrajectories();
+    downloadMembers(d_x, (size_t)nStoreMax * prob.nVar, realSize(), out, cap);
+}
+void Simulator::getDxMembers(double *out, size_t cap)
+{
+    requireTrajectories();
+    downloadMembers(d_dx, (size_t)nStoreMax * prob.nVar, realSize(), out, cap);
+}
+void Simulator::getAuxMembers(double *out, size_t cap)
+{
+    requireTrajectories();
+    downloadMembers(d_aux, (size_t)nStoreMax * prob.nAux, realSize(), out, cap);
+}
 std::vector<int> Simulator::getNstored()
 {
     std::vector<int> out(nPts > 0 ? nPts : 0);

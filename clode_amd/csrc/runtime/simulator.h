@@ -14,6 +14,7 @@
 #include <map>
 
 #include "clode_runtime.h"
+#include "staged_copy.h"
 
 namespace clode {
 
@@ -32,10 +33,10 @@ public:
     void compileOnly();
 
     // data
-    void setProblemData(const std::vector<double> &x0, const std::vector<double> &pars);
+    void setProblemData(const double *x0, size_t nx0, const double *pars, size_t npars);
     void setTspan(const std::vector<double> &t);
-    void setX0(const std::vector<double> &x0);
-    void setPars(const std::vector<double> &pars);
+    void setX0(const double *x0, size_t n);
+    void setPars(const double *pars, size_t n);
     void setSolverParams(const SolverParams &sp);
     void seedRNG();
     void seedRNG(int seed);
@@ -46,11 +47,11 @@ public:
     void shiftTspan();
     void shiftX0();
 
-    // getters
-    std::vector<double> getX0();
-    std::vector<double> getXf();
-    std::vector<double> getDt();
-    std::vector<double> getTf();
+    // getters: into out (capacity cap)
+    void getX0(double *out, size_t cap);
+    void getXf(double *out, size_t cap);
+    void getDt(double *out, size_t cap);
+    void getTf(double *out, size_t cap);
     std::string programString();
 
     // features
@@ -60,18 +61,23 @@ public:
     void features();
     void features(bool reinit);
     void transientFeatures(double tr0, double tr1, double fe0, double fe1);
-    std::vector<double> getF();
-    // F into out (capacity cap): feature-major as getF, or member-major
-    // ([nPts][nF], transposed on the device)
+    // F into out (capacity cap): feature-major, or member-major ([nPts][nF],
+    // transposed on the device)
     void getFInto(double *out, size_t cap);
     void getFMembers(double *out, size_t cap);
 
     // trajectory
     void trajectory();
-    std::vector<double> getT();
-    std::vector<double> getX();
-    std::vector<double> getDx();
-    std::vector<double> getAux();
+    void getT(double *out, size_t cap);
+    void getX(double *out, size_t cap);
+    void getDx(double *out, size_t cap);
+    void getAux(double *out, size_t cap);
+    // the same, member-major: t [nPts][maxStore], x and dx [nPts][maxStore][nVar],
+    // aux [nPts][maxStore][nAux], transposed on the device
+    void getTMembers(double *out, size_t cap);
+    void getXMembers(double *out, size_t cap);
+    void getDxMembers(double *out, size_t cap);
+    void getAuxMembers(double *out, size_t cap);
     std::vector<int> getNstored();
 
     // public state (read by the C ABI)
@@ -85,7 +91,7 @@ public:
     SolverParams sp;
     std::vector<double> tspan{0.0, 1000.0};
     int nPts = 0;
-    std::vector<double> x0, pars, dtHost;
+    std::vector<double> pars, dtHost;
     std::vector<unsigned long long> rngHost;
 
     std::string observer;
@@ -141,7 +147,8 @@ private:
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::shared_ptr<Program> program;
-    std::string programKeyCache;
+    // configGen counts the calls that change what a program is composed from
+    unsigned long long configGen = 0, programGen = ~0ull;
 
     size_t realSize() const { return prec == PREC_DOUBLE ? 8 : 4; }   // pars, trajectory x
     size_t wideSize() const { return prec == PREC_SINGLE ? 4 : 8; }   // x0/xf/dt/tf/F/odata/traj t
@@ -152,21 +159,26 @@ private:
     // default compilation), used by grid launches of large ensembles (see
     // gridFunction), and with the replay kernels when `replay` is set
     std::shared_ptr<Program> variantProgram(int waves, bool replay);
-    std::map<int, std::pair<std::string, std::shared_ptr<Program>>> programsW;
+    std::map<int, std::pair<unsigned long long, std::shared_ptr<Program>>> programsW;
     hipFunction_t gridFunction(const char *kernel, unsigned int nThreads, unsigned int block, bool replay = false);
     void ensureStream();
     void setNpts(int n);
-    void upload(DeviceBuffer &b, const std::vector<double> &v, size_t elem);
-    std::vector<double> download(const DeviceBuffer &b, size_t n, size_t elem);
-    // n elements of b (elem bytes each) as double into out
-    void downloadInto(const DeviceBuffer &b, size_t n, size_t elem, double *out);
-    DeviceBuffer d_Fm;  // member-major copy of F for getFMembers
+    void upload(DeviceBuffer &b, const double *v, size_t n, size_t elem);
+    // n elements of b (elem bytes each) as double into out, cap of them wanted
+    void downloadInto(const DeviceBuffer &b, size_t n, size_t elem, double *out, size_t cap);
+    void toHost(void *dst, const void *src, size_t bytes);
+    // rows x nPts of b (elem bytes each, member index fastest) as double,
+    // member-major, into out
+    void downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out, size_t cap);
+    DeviceBuffer d_members;  // member-major copy of a block of members
+    std::shared_ptr<StagedCopy> staging;
     ClodeArgs makeArgs();
     void launch(const char *kernel, const ClodeArgs &a, unsigned int nThreads, bool replay = false);
     void updateObserverInfo();
     void resizeFeaturesVariables();
     void resizeTrajectoryVariables();
     void requireData(const char *what) const;
+    void requireTrajectories() const;
 };
 
 // resident-workgroup grid for a persistent work-queue launch of fn

@@ -237,7 +237,7 @@ class Simulator:
             unknown = set(spec.keys()) - set(names)
             if unknown:
                 raise ValueError(f"Unknown {what[:-1]} name(s): {unknown}")
-            arrays = {k: np.array(v, dtype=np.float64) for k, v in spec.items()}
+            arrays = {k: np.asarray(v, dtype=np.float64) for k, v in spec.items()}
             shapes = {k: v.shape for k, v in arrays.items() if v.size > 1}
             if len(set(shapes.values())) > 1:
                 raise ValueError(f"Shape of arrays for {what} don't match: {shapes}")
@@ -251,29 +251,26 @@ class Simulator:
                            new_shape: Optional[Tuple] = None):
         if new_shape is None or len(new_shape) == 1:
             new_shape = (new_size, 1)
-        previous = self._ensemble_size
-        if previous == new_size or previous == 1:
-            x0 = np.array(self.get_initial_state(), dtype=np.float64, copy=True)
-            p = np.array(self._device_parameters, dtype=np.float64, copy=True)
-        else:
-            x0 = np.array(list(self._variable_defaults.values()), dtype=np.float64, ndmin=2)
-            p = np.array(list(self._parameter_defaults.values()), dtype=np.float64, ndmin=2)
-        if x0.shape[0] == 1:
-            x0 = np.tile(x0, (new_size, 1))
-        if p.shape[0] == 1:
-            p = np.tile(p, (new_size, 1))
-        if isinstance(variables, np.ndarray):
-            x0 = np.array(variables, dtype=np.float64)
-        elif isinstance(variables, Mapping):
-            for k, v in variables.items():
-                v = np.repeat(v, new_size) if v.size == 1 else v
-                x0[:, self.variable_names.index(k)] = np.asarray(v).flatten()
-        if isinstance(parameters, np.ndarray):
-            p = np.array(parameters, dtype=np.float64)
-        elif isinstance(parameters, Mapping):
-            for k, v in parameters.items():
-                v = np.repeat(v, new_size) if v.size == 1 else v
-                p[:, self.parameter_names.index(k)] = np.asarray(v).flatten()
+        keep = self._ensemble_size in (new_size, 1)
+
+        def fill(spec, names, current, defaults):
+            # column-major, the layout that crosses to the device; columns that
+            # the caller gives are written once
+            if isinstance(spec, np.ndarray):
+                return np.array(spec, dtype=np.float64, order="F")
+            a = np.empty((new_size, len(names)), dtype=np.float64, order="F")
+            given = {names.index(k): v for k, v in (spec or {}).items()}
+            if len(given) < len(names):
+                base = current() if keep else np.array(list(defaults.values()), dtype=np.float64, ndmin=2)
+                for j in range(len(names)):
+                    if j not in given:
+                        a[:, j] = base[:, j]
+            for j, v in given.items():
+                a[:, j] = v.ravel()
+            return a
+
+        x0 = fill(variables, self.variable_names, self.get_initial_state, self._variable_defaults)
+        p = fill(parameters, self.parameter_names, lambda: self._device_parameters, self._parameter_defaults)
         self._ensemble_size = new_size
         self._ensemble_shape = new_shape
         return x0, p
@@ -281,7 +278,7 @@ class Simulator:
     def _set_problem_data(self, initial_state: np.ndarray, parameters: np.ndarray) -> None:
         self._device_initial_state = initial_state
         self._device_parameters = parameters
-        self._integrator.set_problem_data(initial_state.flatten(order="F"), parameters.flatten(order="F"))
+        self._integrator.set_problem_data(initial_state.ravel(order="F"), parameters.ravel(order="F"))
         self._device_final_state = self._device_dt = self._device_tf = None
 
     def _set_parameters(self, parameters: np.ndarray) -> None:

@@ -16,25 +16,43 @@ from .runtime import CLDeviceType, CLVendor, _clode_root_dir
 from .solver import Simulator, Stepper
 
 
+def _struct(names: List[str]) -> np.dtype:
+    return np.dtype({"names": names, "formats": [np.float64] * len(names)})
+
+
 class TrajectoryOutput:
     def __init__(self, t: np.ndarray, x: np.ndarray, dx: np.ndarray, aux: np.ndarray, variable_names: List[str],
                  aux_names: List[str]) -> None:
         self.t = t
-        xdt = np.dtype({"names": variable_names, "formats": [np.float64] * len(variable_names)})
+        xdt = _struct(variable_names)
         self.x = rfn.unstructured_to_structured(np.ascontiguousarray(x), dtype=xdt)
         self.dx = rfn.unstructured_to_structured(np.ascontiguousarray(dx), dtype=xdt)
         if len(aux_names) > 0:
-            adt = np.dtype({"names": aux_names, "formats": [np.float64] * len(aux_names)})
-            self.aux = rfn.unstructured_to_structured(np.ascontiguousarray(aux), dtype=adt)
+            self.aux = rfn.unstructured_to_structured(np.ascontiguousarray(aux), dtype=_struct(aux_names))
         self._variable_names = variable_names
         self._aux_names = aux_names
+
+    @classmethod
+    def _of_structured(cls, t: np.ndarray, x: np.ndarray, dx: np.ndarray, aux: Optional[np.ndarray],
+                       variable_names: List[str], aux_names: List[str]) -> "TrajectoryOutput":
+        """From arrays that are structured already (one member's rows of the ensemble's arrays)."""
+        out = cls.__new__(cls)
+        out.t, out.x, out.dx = t, x, dx
+        if aux is not None:
+            out.aux = aux
+        out._variable_names, out._aux_names = variable_names, aux_names
+        return out
 
     def __repr__(self) -> str:
         return (f"TrajectoryOutput( length: {len(self.t)}, variable names: {self._variable_names}, "
                 f"aux variable names: {self._aux_names} )")
 
     def to_ndarray(self, slot: str, **kwargs) -> np.ndarray:
-        return rfn.structured_to_unstructured(getattr(self, slot), **kwargs)
+        a = getattr(self, slot)
+        if not kwargs and a.flags.c_contiguous and a.dtype.names is not None:
+            # fields of double, one after the other: the same memory as columns
+            return a.view(np.float64).reshape(a.shape + (len(a.dtype.names),))
+        return rfn.structured_to_unstructured(a, **kwargs)
 
 
 class TrajectorySimulator(Simulator):
@@ -97,20 +115,25 @@ class TrajectorySimulator(Simulator):
         return None
 
     def get_trajectory(self):
-        n_stored = np.array(self._integrator.get_n_stored())
         store = self._sp.max_store
-        n, nv, na = self._ensemble_size, self.num_variables, len(self.aux_names)
-        t = np.array(self._integrator.get_t(), dtype=np.float64)[: n * store].reshape((n, store), order="F")
-        x = np.array(self._integrator.get_x(), dtype=np.float64)[: n * nv * store].reshape((n, nv, store),
-                                                                                          order="F")
-        dx = np.array(self._integrator.get_dx(), dtype=np.float64)[: n * nv * store].reshape((n, nv, store),
-                                                                                            order="F")
-        aux = np.array(self._integrator.get_aux(), dtype=np.float64)[: n * na * store].reshape((n, na, store),
-                                                                                              order="F")
-        self._device_t, self._device_x, self._device_dx, self._device_aux = t, x, dx, aux
+        n = self._ensemble_size
+        # every member's samples are rows of one array per kind, transposed to
+        # that order on the device; the members' outputs are slices of them
+        t = self._integrator.get_t_members()
+        if t.shape[1] < store:
+            raise ValueError(f"{t.shape[1]} samples per member are stored, max_store is {store}")
+        t = t[:, :store]
+        x, dx, aux = (get() for get in (self._integrator.get_x_members, self._integrator.get_dx_members,
+                                        self._integrator.get_aux_members))
+        self._device_t = t
+        self._device_x, self._device_dx, self._device_aux = (a.transpose(0, 2, 1)[:, :, :store] for a in (x, dx, aux))
+        names, aux_names = self.variable_names, self.aux_names
+        xs, dxs = (a.view(_struct(names))[..., 0] for a in (x, dx))
+        auxs = aux.view(_struct(aux_names))[..., 0] if len(aux_names) > 0 else None
+        make = TrajectoryOutput._of_structured
         results = []
-        for i in range(n):
-            k = min(int(n_stored[i]) + 1, store)
-            results.append(TrajectoryOutput(t=t[i, :k].T, x=x[i, :, :k].T, dx=dx[i, :, :k].T, aux=aux[i, :, :k].T,
-                                            variable_names=self.variable_names, aux_names=self.aux_names))
+        n_stored = np.array(self._integrator.get_n_stored())
+        for i, k in enumerate(np.minimum(n_stored + 1, store).tolist()):
+            results.append(make(t[i, :k], xs[i, :k], dxs[i, :k], auxs[i, :k] if auxs is not None else None, names,
+                                aux_names))
         return results[0] if n == 1 else results

@@ -190,6 +190,12 @@ int clode_get_t(clode_sim *sim, double *out, size_t n);
 int clode_get_x(clode_sim *sim, double *out, size_t n);
 int clode_get_dx(clode_sim *sim, double *out, size_t n);
 int clode_get_aux(clode_sim *sim, double *out, size_t n);
+/* the same member by member (transposed on the device): t [nPts][max_store],
+ * x and dx [nPts][max_store][num_var], aux [nPts][max_store][num_aux] */
+int clode_get_t_members(clode_sim *sim, double *out, size_t n);
+int clode_get_x_members(clode_sim *sim, double *out, size_t n);
+int clode_get_dx_members(clode_sim *sim, double *out, size_t n);
+int clode_get_aux_members(clode_sim *sim, double *out, size_t n);
 int clode_get_n_stored(clode_sim *sim, int *out, size_t n);
 
 /* ---- logging (CLODEpython.cpp:43-95 LogLevel / get_logger):

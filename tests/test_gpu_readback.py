@@ -1,0 +1,42 @@
+"""Reading trajectories back member by member: the transposition on the device
+(clode_members_f64 / _f32, tiles of 64 members x 32 rows) and the staged copy
+(from 8 MiB on) against the rows as the integrator stores them."""
+
+import os
+
+import numpy as np
+import pytest
+
+import clode_amd as clode
+
+MODELS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "clode_amd", "models")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("n, store", [(1, 5), (63, 32), (64, 33), (65, 31), (257, 1), (5001, 130)])
+def test_members_are_the_stored_rows(gpu_available, n, store, single):
+    rng = np.random.default_rng(n)
+    sim = clode.TrajectorySimulator(src_file=os.path.join(MODELS, "linear_drag.cl"),
+                                    variables={"y1": 0.0, "y2": 0.0},
+                                    parameters={"m": 0.25, "w": 8.0, "k": 2.0, "H": 10.0}, aux=["g1"], num_noise=0,
+                                    dt=0.01, stepper=clode.Stepper.rk4, t_span=(0.0, 0.6), max_store=store,
+                                    max_steps=1000, single_precision=single)
+    sim.set_ensemble(variables={"y1": rng.random(n), "y2": rng.random(n)})
+    out = sim.trajectory()
+    out = [out] if n == 1 else out
+    native = sim._integrator
+    count = np.minimum(np.array(native.get_n_stored()) + 1, store)
+    rows = {}
+    for name, width in (("t", 1), ("x", 2), ("dx", 2), ("aux", 1)):
+        flat = np.array(getattr(native, "get_" + name)())
+        rows[name] = flat[: n * width * store].reshape((n, width, store), order="F")
+    assert len(out) == n
+    for i, tr in enumerate(out):
+        k = count[i]
+        assert np.array_equal(tr.t, rows["t"][i, 0, :k])
+        for j, v in enumerate(("y1", "y2")):
+            assert np.array_equal(tr.x[v], rows["x"][i, j, :k])
+            assert np.array_equal(tr.dx[v], rows["dx"][i, j, :k])
+        assert np.array_equal(tr.aux["g1"], rows["aux"][i, 0, :k])
+        assert np.array_equal(tr.to_ndarray("x"), rows["x"][i, :, :k].T)
