@@ -1075,15 +1075,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
 // One launch for everything of an optimizer step that runs row by row: gather
 // and encode, the four hidden layers, the heads, the loss, and the input
 // gradients back to the first layer.  A workgroup of 8 waves takes 16 rows of
-// the minibatch; activations and gradients stay in LDS (8 KiB), the
-// pre-activations in the registers of the lane that needs them again (a lane
-// forms the same elements of a layer forward and backward), and each wave's
-// weight fragments of the next product are loaded while the current one runs.
-// Only the transposed operands of the weight-gradient products leave the CU.
-// What bounds it is the weights' way from L2: 1 MB per workgroup through the
-// CU's 64 B per cycle, 7 us.  The launches it replaces (gather, five forward
-// products, loss, the input gradients) took about 53 us of GPU time a step at
-// 2048 rows, each waiting for a few hundred workgroups to start and drain.
+// the minibatch; activations and gradients stay in LDS (two 8 KiB tiles, one
+// barrier per layer), SiLU' stays in the registers of the lane that needs it
+// again (a lane forms the same elements of a layer forward and backward), and
+// each wave's weight fragments of the next product are loaded while the current
+// one runs.  Only the transposed operands of the weight-gradient products leave
+// the CU.
+// What bounds it is the chain of nine products, each waiting for the one
+// before: 17 us with 4 workgroups, 21 us with 128 (2048 rows), 23 us with 256;
+// past one workgroup per CU the weights' way from L2, 1 MB per workgroup at
+// 64 B per cycle, 17 us per 256 workgroups.  An optimizer step's three launches
+// take 40 us at 2048 rows and 29 us at 64; the thirteen that this replaces
+// (gather, five forward products, loss, five backward ones, optimizer) took
+// 79 us and 58 us, each waiting for a few hundred workgroups to start and drain.
 // K order and epilogue arithmetic are those of gemm_block, so the weights
 // after training are the same bits.
 constexpr int FROWS = 16;    // rows per workgroup
@@ -1581,8 +1585,8 @@ void backward(clode_mlp *h, int n)
 // output gradients are, for mlp_adam_sum.
 void fused_step(clode_mlp *h, const FusedStep &f, GradSources &gs)
 {
-    hipLaunchKernelGGL(mlp_fused_step, dim3((unsigned int)((f.nb + 8 * FROWS - 1) / (8 * FROWS) * 8)), dim3(FWAVES * 64), 0, h->stream,
-                       f);
+    const unsigned int groups = (unsigned int)((f.nb + 8 * FROWS - 1) / (8 * FROWS) * 8);  // as many for each XCD
+    hipLaunchKernelGGL(mlp_fused_step, dim3(groups), dim3(FWAVES * 64), 0, h->stream, f);
     check(hipGetLastError(), "mlp_fused_step launch");
     WgradAll a;
     int blocks = 0, tiles64 = 0;
@@ -1597,9 +1601,9 @@ void fused_step(clode_mlp *h, const FusedStep &f, GradSources &gs)
             a.g[l].M = NOUT;  // the padding's gradients are not used
         tiles64 += ((a.g[l].N + 63) / 64) * ((a.g[l].M + 63) / 64) * gs.splits;
     }
-    // 32 x 32 tiles until 64 x 64 ones fill every CU twice: a step took 35.4
-    // and 37.7 us with them at 1000 rows (180 tiles of 64 x 64), the same at
-    // 2048 (480), 53.0 and 51.1 at 4096 (960), 175 and 168 at 16384
+    // 32 x 32 tiles until 64 x 64 ones fill every CU twice.  A step took, with
+    // 32 and with 64: 35.4 and 37.7 us at 1000 rows (180 tiles of 64 x 64), the
+    // same at 2048 (480), 53.0 and 51.1 at 4096 (960), 175 and 168 at 16384
     const int tile = tiles64 < 2 * h->cus ? 32 : 64;
     for (int l = 0; l < NLAYER; ++l) {
         a.first[l] = blocks;
