@@ -10,7 +10,6 @@
 
 #include <hip/hiprtc.h>
 
-#include <cctype>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
@@ -226,70 +225,149 @@ void DeviceBuffer::release()
 
 // ------------------------------------------------------------------ program
 
-// The token "/" becomes " *CLODE_DIV* ", which has the same precedence and
-// associativity, so every expression keeps its tree.  Left alone: comments,
-// character and string literals, preprocessor lines (macro bodies keep their
-// divisions), "/=", and everything outside braces.
+// Positions of the division tokens "/" inside the braces of a right-hand side,
+// found as the compiler's lexer finds tokens (C++17, 5.2 to 5.4): line splices
+// first, then comments (which may begin on a preprocessor line and end on a
+// later one), literals, raw strings, numbers with digit separators and names.
+// Not among them: "/=", the "/" of "operator/", everything on preprocessor
+// lines (macro bodies keep their divisions) and everything outside braces.
+// None at all where text could be seen by the program itself: a macro with "#"
+// or "##", assert, or a raw string that does not end.
+static std::vector<size_t> division_tokens(const std::string &rhs)
+{
+    // positions of the characters that remain when line splices are gone
+    std::vector<size_t> at;
+    at.reserve(rhs.size());
+    for (size_t i = 0; i < rhs.size(); ++i) {
+        if (rhs[i] == '\\') {
+            const size_t e = rhs.find_first_not_of(" \t\v\f\r", i + 1);
+            if (e != std::string::npos && rhs[e] == '\n') {
+                i = e;
+                continue;
+            }
+        }
+        at.push_back(i);
+    }
+    const size_t n = at.size();
+    auto ch = [&](size_t k) { return k < n ? rhs[at[k]] : '\0'; };
+    auto digit = [](char c) { return c >= '0' && c <= '9'; };
+    auto name = [&](char c) {
+        return digit(c) || (c >= 'a' && c <= 'z') || (c >= 'A' && c <= 'Z') || c == '_' || c == '$' || (c & 0x80);
+    };
+    std::vector<size_t> out;
+    int depth = 0;
+    bool lineStart = true, directive = false, define = false;
+    std::string last;  // the name just read, if the token before this one is a name
+    for (size_t k = 0; k < n;) {
+        const char c = ch(k), d = ch(k + 1);
+        if (c == '\n') {
+            lineStart = true;
+            directive = define = false;
+            ++k;
+            continue;
+        }
+        if (c == ' ' || c == '\t' || c == '\v' || c == '\f' || c == '\r') {
+            ++k;
+            continue;
+        }
+        if (c == '/' && d == '/') {
+            while (k < n && ch(k) != '\n')
+                ++k;
+            continue;
+        }
+        if (c == '/' && d == '*') {  // a blank, also where it holds line breaks
+            for (k += 2; k < n && !(ch(k) == '*' && ch(k + 1) == '/');)
+                ++k;
+            k = std::min(n, k + 2);
+            continue;
+        }
+        const bool first = lineStart;
+        const std::string before = std::move(last);
+        last.clear();
+        lineStart = false;
+        if (c == '#' || (c == '%' && d == ':')) {
+            if (define)
+                return {};
+            directive = directive || first;
+            k += c == '#' ? 1 : 2;
+            if (first)
+                last = "#";
+            continue;
+        }
+        if (digit(c) || (c == '.' && digit(d))) {
+            for (++k; k < n; ++k) {
+                const char e = ch(k), p = ch(k - 1);
+                const bool sign = (e == '+' || e == '-') && (p == 'e' || p == 'E' || p == 'p' || p == 'P');
+                if (e == '\'' && name(ch(k + 1)))
+                    ++k;
+                else if (!name(e) && e != '.' && !sign)
+                    break;
+            }
+            continue;
+        }
+        if (name(c)) {
+            for (; k < n && name(ch(k)); ++k)
+                last += ch(k);
+            if (ch(k) == '"' && (last == "R" || last == "LR" || last == "uR" || last == "UR" || last == "u8R")) {
+                // as it stands in the text, splices included
+                const size_t open = rhs.find('(', at[k]);
+                if (open == std::string::npos)
+                    return {};
+                const std::string close = ")" + rhs.substr(at[k] + 1, open - at[k] - 1) + "\"";
+                const size_t end = rhs.find(close, open + 1);
+                if (end == std::string::npos)
+                    return {};
+                while (k < n && at[k] < end + close.size())
+                    ++k;
+                last.clear();
+            } else if (last == "assert") {
+                return {};
+            } else if (directive && before == "#") {
+                define = last == "define";
+                if (last == "include" || last == "include_next" || last == "import") {
+                    while (ch(k) == ' ' || ch(k) == '\t')
+                        ++k;
+                    if (ch(k) == '<')  // a file name may hold anything but this
+                        while (k < n && ch(k) != '>' && ch(k) != '\n')
+                            ++k;
+                }
+            }
+            continue;
+        }
+        if (c == '"' || c == '\'') {
+            for (++k; k < n && ch(k) != c && ch(k) != '\n'; ++k)
+                if (ch(k) == '\\' && k + 1 < n)
+                    ++k;
+            if (ch(k) == c)
+                ++k;
+            continue;
+        }
+        if (!directive) {
+            if (c == '{' || (c == '<' && d == '%'))
+                ++depth;
+            else if (c == '}' || (c == '%' && d == '>'))
+                --depth;
+            else if (c == '/' && d != '=' && depth > 0 && before != "operator")
+                out.push_back(at[k]);
+        }
+        ++k;
+    }
+    return out;
+}
+
+// A division token becomes " *CLODE_DIV* ", which has the same precedence and
+// associativity, so every expression keeps its tree; nothing else changes.
 std::string division_operators(const std::string &rhs)
 {
     std::string out;
     out.reserve(rhs.size() + 256);
-    const size_t n = rhs.size();
-    int depth = 0;
-    bool lineStart = true;  // only blanks since the last line break
-    auto spliced = [&](size_t i) {  // the line break at i follows a backslash
-        return (i > 0 && rhs[i - 1] == '\\') || (i > 1 && rhs[i - 1] == '\r' && rhs[i - 2] == '\\');
-    };
-    // up to (not including) the end of the logical line
-    auto copyLine = [&](size_t i) {
-        while (i < n && (rhs[i] != '\n' || spliced(i)))
-            out += rhs[i++];
-        return i;
-    };
-    for (size_t i = 0; i < n;) {
-        const char c = rhs[i], d = i + 1 < n ? rhs[i + 1] : '\0';
-        if (c == '#' && lineStart) {
-            i = copyLine(i);
-            continue;
-        }
-        if (c == '/' && d == '/') {
-            i = copyLine(i);
-            continue;
-        }
-        if (c == '/' && d == '*') {
-            const size_t e = rhs.find("*/", i + 2), stop = e == std::string::npos ? n : e + 2;
-            out.append(rhs, i, stop - i);
-            i = stop;
-            continue;
-        }
-        // a quote starts a literal, except as a digit separator (1'000)
-        if (c == '"' || (c == '\'' && !(i > 0 && (std::isalnum((unsigned char)rhs[i - 1]) || rhs[i - 1] == '_')))) {
-            out += c;
-            for (++i; i < n && rhs[i] != c && rhs[i] != '\n'; ++i) {
-                out += rhs[i];
-                if (rhs[i] == '\\' && i + 1 < n)
-                    out += rhs[++i];
-            }
-            if (i < n)
-                out += rhs[i++];
-            lineStart = false;
-            continue;
-        }
-        if (c == '{')
-            ++depth;
-        else if (c == '}')
-            --depth;
-        if (c == '/' && depth > 0 && d != '=')
-            out += " *CLODE_DIV* ";
-        else
-            out += c;
-        if (c == '\n')
-            lineStart = true;
-        else if (c != ' ' && c != '\t' && c != '\r')
-            lineStart = false;
-        ++i;
+    size_t from = 0;
+    for (size_t i : division_tokens(rhs)) {
+        out.append(rhs, from, i - from);
+        out += " *CLODE_DIV* ";
+        from = i + 1;
     }
-    return out;
+    return out.append(rhs, from, std::string::npos);
 }
 
 // The right-hand side as compiled.  fp32c programs divide by reciprocals

@@ -1,6 +1,7 @@
 """Divisions of a right-hand side (clode_divide.h): which tokens the program builder replaces, that what it cannot
 replace still compiles, and that the quotients by constants are those of IEEE division."""
 import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -43,6 +44,49 @@ def test_outside_functions_as_written(tmp_path):
     text = "const int half = 7 / 2;\n" + HEAD + "dx_[0] = p_[0] / half;\n}\n"
     s = _program(tmp_path, text, False)
     assert "half = 7 / 2;" in s and "p_[0]  *CLODE_DIV*  half" in s
+
+
+# text around divisions that a scanner can take for something else, each a body's lines and its replaced divisions:
+# comments that begin on a preprocessor line, with braces, quotes and division signs in them, literals, spliced lines,
+# numbers, and text that the program itself can see (a stringified argument), which is left alone
+TEXTS = {
+    "comment from a define": ("#define TAU 10.0 /* time constant\n  in ms */\n  dx_[0] = -x_[0];\n"
+                              "  dx_[0] += p_[0] / TAU; /* drive */", 1),
+    "two comments from a define": ("#define K 2 /* a */ /* b\n c\n d */\n dx_[0] = 4.0 / p_[0]; /* c */ aux_[0] = 1;", 1),
+    "comment from a pragma": ("#pragma unroll /* all\n */\n for (int i = 0; i < 2; ++i) dx_[0] = x_[i] / 3; /* e */", 1),
+    "comment from if and endif": ("#if 1 /* on\n */\n dx_[0] = x_[0] / 3;\n#endif /* off\n } */\n aux_[0] = 1 / p_[0];", 2),
+    "braces in the comment": ("#define K 2 /* } } \n { */\n dx_[0] = x_[0] / K;", 1),
+    "quotes in the comment": ("#define K 2 /* it's \"so\n */\n dx_[0] = x_[0] / K; /* ' */ aux_[0] = 1 / p_[0];", 2),
+    "comment before a directive": ("/* a\n b */ #define K (3 / 2)\n dx_[0] = x_[0] / K;", 1),
+    "literal on a directive": ('#define S "/*"\n dx_[0] = x_[0] / 3; /* c */', 1),
+    "skipped lines": ("#if 0\n don't / } \n#endif\n dx_[0] = x_[0] / 3;", 1),
+    "spliced comment": ("dx_[0] = x_[0] /\\\n/ c\n / 3; /\\\n* a / b *\\\n/ aux_[0] = 1 / p_[0];", 2),
+    "spliced string": ('const char *s = "a\\\n/* b"; dx_[0] = x_[0] / 3; /* c */', 1),
+    "raw string": ('const char *s = R"x(a " / )" /* )x"; dx_[0] = x_[0] / 3; /* c */', 1),
+    "numbers": ("dx_[0] = 1'000'0.0/p_[0] + 0x1p-3/x_[0] + 1.e+3/2;", 3),
+    "prefixed literals": ("int c = L'/' + u8'\\'' + '\"'; dx_[0] = c / 3;", 1),
+    "digraphs": ("%:define K 2 /* a\n b */\n <% dx_[0] = x_[0] / K; %>", 1),
+    "stringified argument": ("#define S(x) #x\n const char *s = S(a / b); dx_[0] = x_[0] / 3;", 0),
+    "pasted argument": ("#define S(x) x ## 1\n dx_[0] = x_[0] / 3;", 0),
+}
+
+
+def _tokens(text):
+    out = subprocess.run(["g++", "-E", "-P", "-std=c++17", "-w", "-x", "c++", "-"], input=text, text=True,
+                         capture_output=True, check=True).stdout
+    return "".join(out.split())
+
+
+@pytest.mark.parametrize("text", list(TEXTS))
+def test_same_tokens_as_written(tmp_path, text):
+    """After preprocessing, the composed text differs from the written one in the division token alone."""
+    body, divisions = TEXTS[text]
+    body = HEAD + body + "\n}\n"
+    for precision in (True, False):
+        s = _program(tmp_path, body, precision)
+        s = s[s.index("\n"):s.rindex("#pragma clang force_cuda_host_device end")]
+        assert s.count("*CLODE_DIV*") == divisions
+        assert _tokens(s).replace("*CLODE_DIV*", "/") == _tokens(body)
 
 
 # forms of "/" whose operands or results are not plain real numbers; the last cannot go through the operator (its
@@ -105,6 +149,25 @@ def test_quotients_by_constants(tmp_path, divisor, precision):
     want = want + T(0)  # x = 0 + 1 * (p / c)
     same = (got.view(U) == want.view(U)) | (np.isnan(got) & np.isnan(want))
     assert np.all(same | tie), (p[~(same | tie)][:5], got[~(same | tie)][:5], want[~(same | tie)][:5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [True, False, "fp32c"])
+def test_comments_from_preprocessor_lines(tmp_path, precision):
+    """A model with a comment that begins on a directive gives the states of the same model without comments."""
+    got = []
+    for text in ("#define TAU 10.0 /* time constant\n in ms */\ndx_[0] = -x_[0];\ndx_[0] += p_[0] / TAU; /* drive */\n",
+                 "dx_[0] = -x_[0];\ndx_[0] += p_[0] / 10.0;\n"):
+        path = tmp_path / "c.cl"
+        path.write_text(HEAD + text + "}\n")
+        sim = clode.Simulator(src_file=str(path), variables={"x": 1.0}, parameters={"p": 1.0},
+                              stepper=clode.Stepper.rk4, dt=0.01, t_span=(0.0, 2.0), single_precision=precision)
+        sim.set_ensemble(parameters={"p": np.linspace(0.5, 9.0, 100)})
+        got.append(np.ravel(sim.transient(update_x0=False, fetch_results=True)))
+    assert np.array_equal(got[0], got[1])
+    t = 2.01  # the first time at or past the span's end
+    p = np.linspace(0.5, 9.0, 100) / 10.0
+    np.testing.assert_allclose(got[0], p + (1.0 - p) * np.exp(-t), rtol=0.02)
 
 
 @pytest.mark.gpu
