@@ -100,7 +100,8 @@ constexpr CM_FN Lhs<A> operator*(A a, Tag)
 template <class A, class B>
 constexpr CM_FN auto operator*(Lhs<A> l, B b) -> decltype(l.a / b)
 {
-    return Quotient<Real<decltype(l.a / b)>::fast>::of(l.a, b);
+    // a type of the user's own keeps its operator, also where that gives a real
+    return Quotient<Real<decltype(l.a / b)>::fast && __is_arithmetic(A) && __is_arithmetic(B)>::of(l.a, b);
 }
 
 }  // namespace clode_div

@@ -110,6 +110,35 @@ def test_forms_compile(tmp_path, form, precision):
     _program(tmp_path, HEAD + FORMS[form] + "\n}\n", precision, compile=True)
 
 
+# a type whose own division is not that of the real it converts to
+OWN = "struct R { double v; double operator/(double d) const { return v * d; } CONVERSION };\n"
+
+
+def test_own_type_keeps_its_operator(tmp_path, capfd):
+    """The operator of an own type is called, not its conversion to double (which here cannot be compiled)."""
+    text = OWN.replace("CONVERSION", "template <class T> operator T() const { return typename T::none(0); }")
+    level = clode.get_log_level()
+    clode.set_log_level(clode.LogLevel.debug)
+    try:
+        _program(tmp_path, text + HEAD + "R r{p_[0]}; dx_[0] = r / 3.0;\n}\n", False, compile=True)
+    finally:
+        clode.set_log_level(level)
+    out = "".join(capfd.readouterr())
+    assert "compiled program" in out and "divisions as written" not in out
+
+
+@pytest.mark.gpu
+def test_own_type_value(tmp_path):
+    path = tmp_path / "own.cl"
+    path.write_text(OWN.replace("CONVERSION", "operator double() const { return v; }") + HEAD +
+                    "R r{p_[0]}; dx_[0] = r / 3.0 + r / x_[0];\n}\n")
+    sim = clode.Simulator(src_file=str(path), variables={"x": 2.0}, parameters={"p": 1.0},
+                          stepper=clode.Stepper.euler, dt=1.0, t_span=(0.0, 0.5), single_precision=False)
+    p = np.arange(1.0, 65.0)
+    sim.set_ensemble(parameters={"p": p})
+    assert np.array_equal(np.ravel(sim.transient(update_x0=False, fetch_results=True)), 2.0 + p * 3.0 + p * 2.0)
+
+
 def _quotients(tmp_path, divisor, p, precision):
     """p / divisor as the right-hand side computes it: one Euler step of length 1 from x = 0."""
     path = tmp_path / "q.cl"
