@@ -116,8 +116,11 @@ std::string compose_source(const ProgramConfig &cfg);
 std::string toolchain_identity();
 std::vector<std::string> compile_options(const ProgramConfig &cfg);
 std::shared_ptr<Program> get_program(const ProgramConfig &cfg, const std::string &cache_dir);
+// PROGRAM_FIND: only one that is loaded or cached (else null); PROGRAM_TRY: a
+// failure to compile is not reported as an error
+enum ProgramSearch { PROGRAM_FIND, PROGRAM_TRY, PROGRAM_BUILD };
 std::shared_ptr<Program> get_program_source(const std::string &source, const std::vector<std::string> &options,
-                                            const std::string &cache_dir, bool report = true);
+                                            const std::string &cache_dir, ProgramSearch how = PROGRAM_BUILD);
 
 // batched programs: up to CLODE_BATCH_MAX systems in one code object
 constexpr size_t CLODE_BATCH_MAX = 8;

@@ -678,41 +678,43 @@ static void rtc_check(hiprtcResult r, const char *what)
 }
 
 // A right-hand side that the compiler refuses with its divisions replaced is
-// compiled as written; errors are then those of the user's own text.
-std::shared_ptr<Program> get_program(const ProgramConfig &cfg, const std::string &cache_dir)
+// compiled as written; errors are then those of the user's own text.  A program
+// of the text as written that is there already says that this happened before:
+// it is taken without another attempt at the first.
+static std::shared_ptr<Program> get_either_program(const std::string &source, const std::string &asWritten,
+                                                   const std::vector<std::string> &options,
+                                                   const std::string &cache_dir)
 {
-    ProgramConfig plain = cfg;
-    plain.plainDivision = true;
-    const std::string source = compose_source(cfg), asWritten = compose_source(plain);
     if (source != asWritten) {
+        for (const std::string &s : {source, asWritten})
+            if (auto p = get_program_source(s, options, cache_dir, PROGRAM_FIND))
+                return p;
         try {
-            return get_program_source(source, compile_options(cfg), cache_dir, false);
+            return get_program_source(source, options, cache_dir, PROGRAM_TRY);
         } catch (const RuntimeError &) {
             log_msg(LOG_DEBUG, "right-hand side compiled with its divisions as written");
-        }
-    }
-    return get_program_source(asWritten, compile_options(plain), cache_dir);
-}
-
-std::shared_ptr<Program> get_batch_program(std::vector<ProgramConfig> cfgs, const std::string &cache_dir)
-{
-    const std::string source = compose_batch_source(cfgs);
-    const std::vector<std::string> options = compile_options(cfgs[0]);
-    for (auto &c : cfgs)
-        c.plainDivision = true;
-    const std::string asWritten = compose_batch_source(cfgs);
-    if (source != asWritten) {
-        try {
-            return get_program_source(source, options, cache_dir, false);
-        } catch (const RuntimeError &) {
-            log_msg(LOG_DEBUG, "right-hand sides compiled with their divisions as written");
         }
     }
     return get_program_source(asWritten, options, cache_dir);
 }
 
+std::shared_ptr<Program> get_program(const ProgramConfig &cfg, const std::string &cache_dir)
+{
+    ProgramConfig plain = cfg;
+    plain.plainDivision = true;
+    return get_either_program(compose_source(cfg), compose_source(plain), compile_options(cfg), cache_dir);
+}
+
+std::shared_ptr<Program> get_batch_program(std::vector<ProgramConfig> cfgs, const std::string &cache_dir)
+{
+    const std::string source = compose_batch_source(cfgs);
+    for (auto &c : cfgs)
+        c.plainDivision = true;
+    return get_either_program(source, compose_batch_source(cfgs), compile_options(cfgs[0]), cache_dir);
+}
+
 std::shared_ptr<Program> get_program_source(const std::string &source, const std::vector<std::string> &options,
-                                            const std::string &cache_dir, bool report)
+                                            const std::string &cache_dir, ProgramSearch how)
 {
     auto prog = std::make_shared<Program>();
     prog->source = source;
@@ -728,14 +730,14 @@ std::shared_ptr<Program> get_program_source(const std::string &source, const std
 
     std::lock_guard<std::mutex> lk(g_prog_mu);
     auto it = g_programs.find(key);
-    if (it != g_programs.end() && it->second)
+    if (it != g_programs.end())
         return it->second;
-    if (it != g_programs.end() && !report)  // known to fail
-        throw RuntimeError("hipRTC build failed");
 
     const std::string path = cache_dir.empty() ? std::string() : cache_path(cache_dir, key);
     if (!path.empty() && read_cache(path, key, prog->code)) {
         log_msg(LOG_DEBUG, "loaded cached code object " + path);
+    } else if (how == PROGRAM_FIND) {
+        return nullptr;
     } else {
         std::vector<const char *> hdrs, names;
         for (const auto &h : kDeviceSources) {
@@ -757,9 +759,7 @@ std::shared_ptr<Program> get_program_source(const std::string &source, const std
             hiprtcGetProgramLog(p, &buildlog[0]);
         if (r != HIPRTC_SUCCESS) {
             hiprtcDestroyProgram(&p);
-            if (!report)
-                g_programs[key] = nullptr;
-            log_msg(report ? LOG_ERR : LOG_DEBUG, "hipRTC build failed:\n" + buildlog);
+            log_msg(how == PROGRAM_TRY ? LOG_DEBUG : LOG_ERR, "hipRTC build failed:\n" + buildlog);
             throw RuntimeError("hipRTC build failed: " + buildlog);
         }
         if (logsize > 1)

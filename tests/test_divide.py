@@ -110,6 +110,26 @@ def test_forms_compile(tmp_path, form, precision):
     _program(tmp_path, HEAD + FORMS[form] + "\n}\n", precision, compile=True)
 
 
+def test_fallback_is_compiled_once(tmp_path):
+    """A text that compiles only as written comes from the cache in the next process, with no attempt at the other."""
+    script = tmp_path / "compile.py"
+    script.write_text(f"""
+import sys
+sys.path.insert(0, {os.path.dirname(os.path.dirname(os.path.abspath(__file__)))!r})
+import clode_amd as clode
+from clode_amd.cpp import clode_cpp_wrapper as w
+clode.set_log_level(clode.LogLevel.debug)
+pi = w.ProblemInfo({str(tmp_path / "rhs.cl")!r}, ["x"], ["p"], [], 0)
+for _ in range(2):
+    w.SimulatorBase(pi, "euler", False, w.OpenCLResource(), {str(tmp_path / "cache")!r}).compile()
+""")
+    (tmp_path / "rhs.cl").write_text(HEAD + FORMS["own type"] + "\n}\n")
+    logs = [subprocess.run(["python3", str(script)], capture_output=True, text=True, check=True) for _ in range(2)]
+    first, second = (r.stdout + r.stderr for r in logs)
+    assert first.count("divisions as written") == 1 and first.count("compiled program") == 1
+    assert "build failed" not in second and "compiled program" not in second and second.count("loaded cached code") == 1
+
+
 # a type whose own division is not that of the real it converts to
 OWN = "struct R { double v; double operator/(double d) const { return v * d; } CONVERSION };\n"
 
