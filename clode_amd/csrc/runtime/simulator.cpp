@@ -276,9 +276,9 @@ static void require_capacity(size_t cap, size_t n)
 void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, double *out, size_t cap)
 {
     require_capacity(cap, n);
-    ensureStream();
-    if (n == 0)
+    if (n == 0)  // nothing set yet: no device is needed
         return;
+    ensureStream();
     if (!b.ptr) {
         std::fill(out, out + n, 0.0);
         return;

@@ -8,8 +8,17 @@ import numpy as np
 import pytest
 
 import clode_amd as clode
+from clode_amd.cpp import clode_cpp_wrapper as w
 
 MODELS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "clode_amd", "models")
+
+
+def test_getters_before_any_data():
+    """Empty results before problem data are set, also where there is no device."""
+    pi = w.ProblemInfo(os.path.join(MODELS, "van_der_pol.cl"), ["x", "y"], ["mu"], [], 0)
+    sim = w.TrajectorySimulatorBase(pi, "rk4", False, w.OpenCLResource(), "")
+    for name in ("x0", "xf", "dt", "tf", "t_members", "x_members", "dx_members", "aux_members"):
+        assert np.size(getattr(sim, "get_" + name)()) == 0
 
 
 @pytest.mark.gpu
