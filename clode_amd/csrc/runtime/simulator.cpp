@@ -96,7 +96,7 @@ void Simulator::setPrecision(int p)
         nPts = 0;
         Felements = 0;
         nStoreMax = 0;
-        telements = 0;
+        telements = xelements = auxelements = 0;
         observerInitialized = false;
     }
 }
@@ -118,7 +118,7 @@ void Simulator::setDevice(int d)
         nPts = 0;
         Felements = 0;
         nStoreMax = 0;
-        telements = 0;
+        telements = xelements = auxelements = 0;
         observerInitialized = false;
     }
 }
@@ -267,6 +267,16 @@ void Simulator::toHost(void *dst, const void *src, size_t bytes)
     hip_check(staging->toHost(device, dst, src, bytes, stream), "hipMemcpy D2H");
 }
 
+// The buffers keep the sizes they were made with when the problem's dimensions
+// change; nothing is read or written past them.
+static bool holds(const DeviceBuffer &b, size_t bytes) { return b.ptr && b.bytes >= bytes; }
+
+static void require_size(const DeviceBuffer &b, size_t bytes)
+{
+    if (!holds(b, bytes))
+        throw InvalidArgument("the data on the device are those of a problem of other dimensions");
+}
+
 static void require_capacity(size_t cap, size_t n)
 {
     if (cap < n)
@@ -283,6 +293,7 @@ void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, doubl
         std::fill(out, out + n, 0.0);
         return;
     }
+    require_size(b, n * elem);
     if (elem == 8) {
         toHost(out, b.ptr, n * 8);
     } else {
@@ -305,6 +316,7 @@ void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem,
         std::fill(out, out + n * rows, 0.0);
         return;
     }
+    require_size(b, n * rows * elem);
     ensureStream();
     size_t block = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (rows * 8)));
     while (!d_members.ptr || d_members.device != device || d_members.bytes < block * rows * 8) {
@@ -337,7 +349,7 @@ void Simulator::setNpts(int newNpts)
     ++inputGen;
     if (newNpts <= 0)
         throw InvalidArgument("the ensemble must have at least one member");
-    if (newNpts == nPts)
+    if (newNpts == nPts && problemDataFit())
         return;
     set_device(device);
     size_t total = 0, freeb = 0;
@@ -396,6 +408,7 @@ void Simulator::setX0(const double *nx0, size_t n)
 {
     ++inputGen;
     if (nPts > 0 && n == (size_t)nPts * prob.nVar) {
+        require_size(d_x0, n * wideSize());
         upload(d_x0, nx0, n, wideSize());
     } else {
         log_msg(LOG_INFO, "...Initial conditions were not updated!");
@@ -407,6 +420,7 @@ void Simulator::setPars(const double *np, size_t n)
 {
     ++inputGen;
     if (nPts > 0 && n == (size_t)nPts * prob.nPar) {
+        require_size(d_pars, n * realSize());
         pars.assign(np, np + n);
         upload(d_pars, np, n, realSize());
     } else {
@@ -508,6 +522,15 @@ void Simulator::requireData(const char *what) const
 {
     if (nPts <= 0)
         throw InvalidArgument(std::string(what) + ": problem data (x0, pars) must be set first");
+    if (!problemDataFit())
+        throw InvalidArgument(std::string(what) + ": problem data (x0, pars) must be set again for these dimensions");
+}
+
+bool Simulator::problemDataFit() const
+{
+    const size_t n = (size_t)nPts, nx = n * prob.nVar * wideSize();
+    return holds(d_x0, nx) && holds(d_xf, nx) && holds(d_pars, n * prob.nPar * realSize()) &&
+           holds(d_rng, n * 16) && holds(d_dt, n * wideSize()) && holds(d_tf, n * wideSize());
 }
 
 ClodeArgs Simulator::makeArgs()
@@ -739,7 +762,8 @@ void Simulator::resizeFeaturesVariables()
     size_t nr = (size_t)clode_obs_nreal(obs, prob.nVar, prob.nAux, S);
     size_t nu = (size_t)clode_obs_nuint(obs);
     size_t fe = (size_t)nFeatures * nPts;
-    if (fe != Felements || nr != odrFields || nu != oduFields || !d_F.ptr) {
+    if (fe != Felements || nr != odrFields || nu != oduFields || !holds(d_odr, nr * nPts * wideSize()) ||
+        !holds(d_odu, nu * nPts * 4) || !holds(d_F, fe * wideSize())) {
         Felements = fe;
         odrFields = nr;
         oduFields = nu;
@@ -911,12 +935,15 @@ void Simulator::resizeTrajectoryVariables()
     hipMemGetInfo(&freeb, &total);
     if (total && largest > total)
         throw InvalidArgument("nPts*nStoreMax*nVar*realSize or nPts*nStoreMax*nAux*realSize is too big");
-    size_t te = (size_t)store * nPts;
-    if (nStoreMax != store || telements != te || !d_t.ptr) {
+    const size_t te = (size_t)store * nPts, xe = (size_t)prob.nVar * te;
+    const size_t ae = prob.nAux > 0 ? (size_t)prob.nAux * te : 1;
+    if (nStoreMax != store || telements != te || xelements != xe || auxelements != ae ||
+        !holds(d_t, te * wideSize()) || !holds(d_x, xe * realSize()) || !holds(d_dx, xe * realSize()) ||
+        !holds(d_aux, ae * realSize()) || !holds(d_nStored, (size_t)nPts * 4)) {
         nStoreMax = store;
         telements = te;
-        xelements = (size_t)prob.nVar * te;
-        auxelements = prob.nAux > 0 ? (size_t)prob.nAux * te : 1;
+        xelements = xe;
+        auxelements = ae;
         d_t.allocate(device, te * wideSize());
         d_x.allocate(device, xelements * realSize());
         d_dx.allocate(device, xelements * realSize());
@@ -939,36 +966,38 @@ void Simulator::getT(double *out, size_t cap) { downloadInto(d_t, telements, wid
 void Simulator::getX(double *out, size_t cap) { downloadInto(d_x, xelements, realSize(), out, cap); }
 void Simulator::getDx(double *out, size_t cap) { downloadInto(d_dx, xelements, realSize(), out, cap); }
 void Simulator::getAux(double *out, size_t cap) { downloadInto(d_aux, auxelements, realSize(), out, cap); }
-void Simulator::requireTrajectories() const
+// rows of the stored trajectories as they were made, `width` values per sample
+size_t Simulator::storedRows(size_t elements, int width) const
 {
-    if (telements != (size_t)nStoreMax * (size_t)(nPts > 0 ? nPts : 0))
+    const size_t te = (size_t)nStoreMax * (size_t)(nPts > 0 ? nPts : 0);
+    if (telements != te)
         throw InvalidArgument("the stored trajectories are those of another ensemble size");
+    if (te > 0 && width > 0 && elements != te * width)
+        throw InvalidArgument("the stored trajectories are those of a problem of other dimensions");
+    return (size_t)nStoreMax * width;
 }
 void Simulator::getTMembers(double *out, size_t cap)
 {
-    requireTrajectories();
-    downloadMembers(d_t, nStoreMax, wideSize(), out, cap);
+    downloadMembers(d_t, storedRows(telements, 1), wideSize(), out, cap);
 }
 void Simulator::getXMembers(double *out, size_t cap)
 {
-    requireTrajectories();
-    downloadMembers(d_x, (size_t)nStoreMax * prob.nVar, realSize(), out, cap);
+    downloadMembers(d_x, storedRows(xelements, prob.nVar), realSize(), out, cap);
 }
 void Simulator::getDxMembers(double *out, size_t cap)
 {
-    requireTrajectories();
-    downloadMembers(d_dx, (size_t)nStoreMax * prob.nVar, realSize(), out, cap);
+    downloadMembers(d_dx, storedRows(xelements, prob.nVar), realSize(), out, cap);
 }
 void Simulator::getAuxMembers(double *out, size_t cap)
 {
-    requireTrajectories();
-    downloadMembers(d_aux, (size_t)nStoreMax * prob.nAux, realSize(), out, cap);
+    downloadMembers(d_aux, storedRows(auxelements, prob.nAux), realSize(), out, cap);
 }
 std::vector<int> Simulator::getNstored()
 {
     std::vector<int> out(nPts > 0 ? nPts : 0);
     if (!d_nStored.ptr || out.empty())
         return out;
+    require_size(d_nStored, out.size() * 4);
     ensureStream();
     hip_check(hipMemcpyAsync(out.data(), d_nStored.ptr, out.size() * 4, hipMemcpyDeviceToHost, stream),
               "hipMemcpy D2H");

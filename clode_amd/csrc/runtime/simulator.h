@@ -178,7 +178,8 @@ private:
     void resizeFeaturesVariables();
     void resizeTrajectoryVariables();
     void requireData(const char *what) const;
-    void requireTrajectories() const;
+    bool problemDataFit() const;
+    size_t storedRows(size_t elements, int width) const;
 };
 
 // resident-workgroup grid for a persistent work-queue launch of fn

@@ -49,3 +49,43 @@ def test_members_are_the_stored_rows(gpu_available, n, store, single):
             assert np.array_equal(tr.dx[v], rows["dx"][i, j, :k])
         assert np.array_equal(tr.aux["g1"], rows["aux"][i, 0, :k])
         assert np.array_equal(tr.to_ndarray("x"), rows["x"][i, :, :k].T)
+
+
+def _native(model, variables, parameters, aux, x0, pars, store):
+    pi = w.ProblemInfo(os.path.join(MODELS, model), variables, parameters, aux, 0)
+    sim = w.TrajectorySimulatorBase(pi, "rk4", False, w.OpenCLResource(), "")
+    sim.set_solver_params(w.SolverParams(0.01, 1.0, 1e-6, 1e-4, 1000, store, 1))  # the step of data set after it
+    sim.set_problem_data(x0.ravel(order="F"), pars.ravel(order="F"))
+    sim.set_tspan([0.0, 0.5])
+    sim.trajectory()
+    return sim
+
+
+@pytest.mark.gpu
+def test_data_of_another_problem_are_not_read(gpu_available):
+    """A problem with more variables and aux outputs: what is on the device is refused until it is set or integrated
+    again, by getters and launches alike, and then has the new sizes."""
+    n, store = 65, 33
+    rng = np.random.default_rng(5)
+    vdp = ("van_der_pol.cl", ["x", "y"], ["mu"], [], rng.random((n, 2)), rng.random((n, 1)), store)
+    drag = ("linear_drag.cl", ["y1", "y2"], ["m", "w", "k", "H"], ["g1"], rng.random((n, 2)), 1 + rng.random((n, 4)), store)
+    lorenz = ("lorenz.cl", ["x", "y", "z"], ["r", "s", "b"], [], rng.random((n, 3)), 1 + rng.random((n, 3)), store)
+    for second in (drag, lorenz):
+        sim = _native(*vdp)
+        sim.set_problem_info(w.ProblemInfo(os.path.join(MODELS, second[0]), second[1], second[2], second[3], 0))
+        for name in ("aux_members",) if second is drag else ("x_members", "dx_members"):
+            with pytest.raises(ValueError):
+                getattr(sim, "get_" + name)()
+        if len(second[1]) > 2:
+            with pytest.raises(ValueError):
+                sim.get_x0()
+            with pytest.raises(ValueError):
+                sim.set_x0(second[4].ravel(order="F"))
+        for call in (sim.transient, sim.trajectory, sim.shift_x0):
+            with pytest.raises(ValueError):
+                call()
+        sim.set_problem_data(second[4].ravel(order="F"), second[5].ravel(order="F"))
+        sim.trajectory()
+        fresh = _native(*second)
+        for name in ("t_members", "x_members", "dx_members", "aux_members", "n_stored", "xf"):
+            assert np.array_equal(getattr(sim, "get_" + name)(), getattr(fresh, "get_" + name)())
