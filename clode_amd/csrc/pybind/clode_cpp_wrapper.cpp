@@ -556,10 +556,9 @@ public:
         sizes(nt, nx, na);
         const py::ssize_t n = (py::ssize_t)n_pts(), store = n > 0 ? (py::ssize_t)nt / n : 0;
         DArray v = k < 0 ? DArray({n, store}) : DArray({n, store, k});
-        {
-            py::gil_scoped_release nogil;
-            check(get(sim_, v.mutable_data(), (size_t)v.size()));
-        }
+        // like the other trajectory getters with the interpreter lock held, so
+        // that no other thread changes the simulator meanwhile
+        check(get(sim_, v.mutable_data(), (size_t)v.size()));
         return v;
     }
     DArray get_t_members() { return members(clode_get_t_members, -1); }

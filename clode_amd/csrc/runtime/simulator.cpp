@@ -262,8 +262,6 @@ void Simulator::upload(DeviceBuffer &b, const double *v, size_t n, size_t elem)
 
 void Simulator::toHost(void *dst, const void *src, size_t bytes)
 {
-    if (!staging)
-        staging = StagedCopy::get();
     hip_check(staging->toHost(device, dst, src, bytes, stream), "hipMemcpy D2H");
 }
 
@@ -317,6 +315,7 @@ void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem,
         return;
     }
     require_size(b, n * rows * elem);
+    std::lock_guard<std::mutex> lk(membersMu);
     ensureStream();
     size_t block = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (rows * 8)));
     while (!d_members.ptr || d_members.device != device || d_members.bytes < block * rows * 8) {

@@ -12,6 +12,7 @@
 #pragma once
 
 #include <map>
+#include <mutex>
 
 #include "clode_runtime.h"
 #include "staged_copy.h"
@@ -170,8 +171,9 @@ private:
     // rows x nPts of b (elem bytes each, member index fastest) as double,
     // member-major, into out
     void downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out, size_t cap);
-    DeviceBuffer d_members;  // member-major copy of a block of members
-    std::shared_ptr<StagedCopy> staging;
+    DeviceBuffer d_members;  // member-major copy of a block of members, one reader's at a time
+    std::mutex membersMu;
+    const std::shared_ptr<StagedCopy> staging = StagedCopy::get();
     ClodeArgs makeArgs();
     void launch(const char *kernel, const ClodeArgs &a, unsigned int nThreads, bool replay = false);
     void updateObserverInfo();

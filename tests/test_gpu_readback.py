@@ -3,6 +3,7 @@
 (from 8 MiB on) against the rows as the integrator stores them."""
 
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -89,3 +90,32 @@ def test_data_of_another_problem_are_not_read(gpu_available):
         fresh = _native(*second)
         for name in ("t_members", "x_members", "dx_members", "aux_members", "n_stored", "xf"):
             assert np.array_equal(getattr(sim, "get_" + name)(), getattr(fresh, "get_" + name)())
+
+
+@pytest.mark.gpu
+def test_two_threads_read_one_simulator(gpu_available):
+    """Threads that read one simulator at the same time get what each gets alone: trajectories, and the feature matrix,
+    whose getter gives up the interpreter lock."""
+    n, store = 4099, 67
+    rng = np.random.default_rng(6)
+    sim = _native("lorenz.cl", ["x", "y", "z"], ["r", "s", "b"], [], rng.random((n, 3)), 1 + rng.random((n, 3)), store)
+    pi = w.ProblemInfo(os.path.join(MODELS, "lorenz.cl"), ["x", "y", "z"], ["r", "s", "b"], [], 0)
+    feat = w.FeatureSimulatorBase(pi, "rk4", "basicall", w.ObserverParams(), True, w.OpenCLResource(), "")
+    feat.set_problem_data(rng.random(3 * n), 1 + rng.random(3 * n))
+    feat.set_tspan([0.0, 0.5])
+    feat.features()
+    calls = [sim.get_t_members, sim.get_x_members, sim.get_dx_members, sim.get_xf] + 4 * [feat.get_f_members]
+    alone = [np.array(call()) for call in calls]
+    wrong = []
+
+    def read(k):
+        for _ in range(12):
+            if not np.array_equal(calls[k](), alone[k], equal_nan=True):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
