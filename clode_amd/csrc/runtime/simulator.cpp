@@ -301,12 +301,25 @@ void Simulator::downloadInto(const DeviceBuffer &b, size_t n, size_t elem, doubl
     }
 }
 
+// Device memory that a read-back may take beside the data.
+// CLODE_MEMBERS_BYTES in the environment replaces the 256 MiB.
+static size_t members_limit()
+{
+    const char *e = std::getenv("CLODE_MEMBERS_BYTES");
+    return e ? (size_t)std::strtoull(e, nullptr, 10) : (size_t)256 << 20;
+}
+
 // The transposition runs on the device (clode_members_*), a block of members
-// at a time so that the copy takes at most 256 MiB beside the data (one
-// member's rows where those are more).
+// at a time so that the copy takes at most members_limit() beside the data.
+// Where not even one member fits, or the device has no memory left, the rows
+// are taken apart on the host; for one member they are the result already.
 void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out, size_t cap)
 {
     const size_t n = nPts > 0 ? (size_t)nPts : 0;
+    if (n == 1) {
+        downloadInto(b, rows, elem, out, cap);
+        return;
+    }
     require_capacity(cap, n * rows);
     if (n * rows == 0)
         return;
@@ -317,16 +330,18 @@ void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem,
     require_size(b, n * rows * elem);
     std::lock_guard<std::mutex> lk(membersMu);
     ensureStream();
-    size_t block = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (rows * 8)));
-    while (!d_members.ptr || d_members.device != device || d_members.bytes < block * rows * 8) {
+    size_t block = std::min(n, members_limit() / (rows * 8));
+    while (block > 0 && (d_members.device != device || !holds(d_members, block * rows * 8))) {
         try {
             d_members.allocate(device, block * rows * 8);
         } catch (const std::exception &) {  // a nearly full device: smaller blocks
             (void)hipGetLastError();
-            if (block == 1)
-                throw;
             block /= 2;
         }
+    }
+    if (block == 0) {
+        hostMembers(b, rows, elem, out);
+        return;
     }
     hipFunction_t fn = currentProgram()->function(device, elem == 8 ? "clode_members_f64" : "clode_members_f32");
     for (size_t m0 = 0; m0 < n; m0 += block) {
@@ -339,6 +354,21 @@ void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem,
         const unsigned int grid = (unsigned int)std::min<unsigned long long>(tiles, 1u << 20);
         hip_check(hipModuleLaunchKernel(fn, grid, 1, 1, 64, 1, 1, 0, stream, params, nullptr), "launch clode_members");
         toHost(out + m0 * rows, d_members.ptr, (size_t)count * rows * 8);
+    }
+}
+
+void Simulator::hostMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out)
+{
+    const size_t n = (size_t)nPts, chunk = std::max<size_t>(1, std::min(rows, ((size_t)16 << 20) / (n * elem)));
+    std::vector<double> part((chunk * n * elem + 7) / 8);
+    for (size_t r0 = 0; r0 < rows; r0 += chunk) {
+        const size_t k = std::min(chunk, rows - r0);
+        toHost(part.data(), b.as<char>() + r0 * n * elem, k * n * elem);
+        const double *d = part.data();
+        const float *f = reinterpret_cast<const float *>(d);
+        for (size_t m = 0; m < n; ++m)
+            for (size_t r = 0; r < k; ++r)
+                out[m * rows + r0 + r] = elem == 8 ? d[r * n + m] : (double)f[r * n + m];
     }
 }
 
@@ -372,6 +402,7 @@ void Simulator::setNpts(int newNpts)
     d_tspan_m.release();
     d_qorder.release();
     d_steps.release();
+    d_members.release();
     seedRNG();
     log_msg(LOG_DEBUG, "set nPts=" + std::to_string(nPts));
 }
@@ -766,6 +797,7 @@ void Simulator::resizeFeaturesVariables()
         Felements = fe;
         odrFields = nr;
         oduFields = nu;
+        d_members.release();
         d_odr.allocate(device, nr * nPts * wideSize());
         d_odu.allocate(device, nu * nPts * 4);
         d_F.allocate(device, fe * wideSize());
@@ -943,6 +975,7 @@ void Simulator::resizeTrajectoryVariables()
         telements = te;
         xelements = xe;
         auxelements = ae;
+        d_members.release();  // the new arrays may need the room
         d_t.allocate(device, te * wideSize());
         d_x.allocate(device, xelements * realSize());
         d_dx.allocate(device, xelements * realSize());

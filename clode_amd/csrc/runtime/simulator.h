@@ -171,6 +171,7 @@ private:
     // rows x nPts of b (elem bytes each, member index fastest) as double,
     // member-major, into out
     void downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out, size_t cap);
+    void hostMembers(const DeviceBuffer &b, size_t rows, size_t elem, double *out);
     DeviceBuffer d_members;  // member-major copy of a block of members, one reader's at a time
     std::mutex membersMu;
     const std::shared_ptr<StagedCopy> staging = StagedCopy::get();

@@ -24,6 +24,17 @@ def test_getters_before_any_data():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("members", [0, 1, 5, 70, 200])
+def test_members_block_by_block(gpu_available, monkeypatch, members, single):
+    """Read-back in blocks of a few members (the last one smaller; 0: not even one member fits, and the host takes the
+    rows apart), blocks that differ from kind to kind, and one that stays for the next read."""
+    n, store = 257, 67
+    monkeypatch.setenv("CLODE_MEMBERS_BYTES", str(members * store * 2 * 8))
+    test_members_are_the_stored_rows(None, n, store, single)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("single", [False, True])
 @pytest.mark.parametrize("n, store", [(1, 5), (63, 32), (64, 33), (65, 31), (257, 1), (5001, 130)])
 def test_members_are_the_stored_rows(gpu_available, n, store, single):
     rng = np.random.default_rng(n)
