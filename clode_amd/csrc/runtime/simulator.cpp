@@ -343,7 +343,10 @@ void Simulator::downloadMembers(const DeviceBuffer &b, size_t rows, size_t elem,
         hostMembers(b, rows, elem, out);
         return;
     }
-    hipFunction_t fn = currentProgram()->function(device, elem == 8 ? "clode_members_f64" : "clode_members_f32");
+    // these kernels are the same in every program: one that is loaded does,
+    // also if it is not the one that the next launch needs
+    const std::shared_ptr<Program> p = program ? program : currentProgram();
+    hipFunction_t fn = p->function(device, elem == 8 ? "clode_members_f64" : "clode_members_f32");
     for (size_t m0 = 0; m0 < n; m0 += block) {
         const void *src = b.ptr;
         void *dst = d_members.ptr;

@@ -34,6 +34,22 @@ def test_members_block_by_block(gpu_available, monkeypatch, members, single):
 
 
 @pytest.mark.gpu
+def test_reading_compiles_nothing(gpu_available, capfd):
+    """Trajectories are read after the simulator was configured for another program, which is not compiled for it."""
+    sim = _native("van_der_pol.cl", ["x", "y"], ["mu"], [], np.ones((3, 2)), np.ones((3, 1)), 7)
+    x = sim.get_x_members()
+    sim.set_stepper("heun")
+    level = clode.get_log_level()
+    clode.set_log_level(clode.LogLevel.debug)
+    try:
+        again = sim.get_x_members()
+    finally:
+        clode.set_log_level(level)
+    assert np.array_equal(x, again)
+    assert "compiled" not in "".join(capfd.readouterr())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("single", [False, True])
 @pytest.mark.parametrize("n, store", [(1, 5), (63, 32), (64, 33), (65, 31), (257, 1), (5001, 130)])
 def test_members_are_the_stored_rows(gpu_available, n, store, single):
