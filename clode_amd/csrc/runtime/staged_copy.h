@@ -117,6 +117,10 @@ private:
         work(0);
         for (auto &t : helpers)
             t.join();
+        // after an error a copy into a block may still be on its way, and the
+        // blocks are free for the next caller from here on
+        if (error.load() != hipSuccess)
+            (void)hipStreamSynchronize(stream);
         return (hipError_t)error.load();
     }
 
