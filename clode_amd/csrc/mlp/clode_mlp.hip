@@ -1391,11 +1391,13 @@ struct clode_mlp {
     double lastMs = 0;
     size_t rows = 0;
     unsigned char *stage = nullptr;  // this device's static scratch (no-allocation screening)
-    // outputs of the last screening, kept for the next up to GRID_KEEP cells
+    // outputs of the last screening, kept for the next up to GRID_KEEP cells;
+    // one screening of a network uses them at a time
+    std::mutex gridMu;
     Dev<float> gP, gA;
     Dev<int> gC;
     Dev<uint8_t> gF, gF2;
-    std::shared_ptr<clode::StagedCopy> staging;
+    const std::shared_ptr<clode::StagedCopy> staging = clode::StagedCopy::get();
 
     WeightCopies copies() const { return {pbf.p, pbfT.p, pbfF.p, pbfTF.p}; }
     LayerTable table() const
@@ -1632,8 +1634,6 @@ void upload(clode_mlp *h, void *dst, const void *src, size_t bytes)
 }
 void download(clode_mlp *h, void *dst, const void *src, size_t bytes)
 {
-    if (!h->staging)
-        h->staging = clode::StagedCopy::get();
     check(h->staging->toHost(h->device, dst, src, bytes, h->stream), "hipMemcpy D2H");
 }
 
@@ -2165,6 +2165,7 @@ int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, f
     need(flags, "flags output");
     check(hipSetDevice(h->device), "hipSetDevice");
     const long long ncell = (long long)nx * ny;
+    std::lock_guard<std::mutex> lk(h->gridMu);
     // the fused kernel by default; CLODE_MLP_FUSED_SCREEN=0 runs the network
     // layer by layer over chunks of 2^18 cells (same results, bit for bit)
     const char *fe = std::getenv("CLODE_MLP_FUSED_SCREEN");

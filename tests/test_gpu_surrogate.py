@@ -9,6 +9,7 @@ change propagates); gradients agree to 1 % in norm per layer with cosine
 > 0.9999.  A transposed or misindexed operand gives O(1) errors.
 """
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -221,6 +222,27 @@ def test_screen_fused_matches_layer_by_layer(gpu_available, shape):
         assert a.shape == (nx, ny)
         assert np.array_equal(a, b)
     assert np.all(np.isfinite(fused[0])) and np.all(np.isfinite(fused[1]))
+
+
+def test_two_threads_screen_one_network(gpu_available):
+    """Threads that screen different grids with one network at the same time get what each gets alone."""
+    m = net(6)
+    grids = [(37, 11), (700, 900), (1200, 1300), (64, 64)]
+    alone = [m.screen_grid(*g, tol=0.05, dilate=1) for g in grids]
+    wrong = []
+
+    def screen(k):
+        for _ in range(5):
+            out = m.screen_grid(*grids[k], tol=0.05, dilate=1)
+            if not all(np.array_equal(a, b, equal_nan=a.dtype.kind == "f") for a, b in zip(out, alone[k])):
+                wrong.append(grids[k])
+
+    threads = [threading.Thread(target=screen, args=(k,)) for k in range(len(grids))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
 
 
 @pytest.mark.parametrize("heads", ["all classes tie", "ties across the halves", "far apart", "infinite"])
