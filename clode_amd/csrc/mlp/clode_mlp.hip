@@ -2176,6 +2176,20 @@ int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, f
     Dev<float> &dP = h->gP, &dA = h->gA;
     Dev<int> &dC = h->gC;
     Dev<uint8_t> &dF = h->gF, &dF2 = h->gF2;
+    struct GiveBack {  // a grid past GRID_KEEP leaves nothing behind, nor does a call that fails
+        clode_mlp *h;
+        bool keep;
+        ~GiveBack()
+        {
+            if (keep)
+                return;
+            h->gP.free();
+            h->gA.free();
+            h->gC.free();
+            h->gF.free();
+            h->gF2.free();
+        }
+    } back{h, false};
     dP.alloc(ncell);
     dA.alloc(ncell);
     dC.alloc(ncell);
@@ -2204,13 +2218,7 @@ int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, f
     float ms = 0;
     (void)hipEventElapsedTime(&ms, h->ev0, h->ev1);
     h->lastMs = ms;
-    if (ncell > GRID_KEEP) {  // a grid this large is given back at once
-        dP.free();
-        dA.free();
-        dC.free();
-        dF.free();
-        dF2.free();
-    }
+    back.keep = ncell <= GRID_KEEP;
     MLP_CATCH
 }
 

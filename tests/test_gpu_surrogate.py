@@ -8,6 +8,7 @@ side of a BF16 rounding boundary, one activation moves by a BF16 ulp and the
 change propagates); gradients agree to 1 % in norm per layer with cosine
 > 0.9999.  A transposed or misindexed operand gives O(1) errors.
 """
+import ctypes
 import os
 import threading
 
@@ -243,6 +244,22 @@ def test_two_threads_screen_one_network(gpu_available):
     for t in threads:
         t.join()
     assert wrong == []
+
+
+def test_large_grid_is_given_back(gpu_available):
+    """Screening more cells than are kept leaves no more device memory in use than a small screening."""
+    hip = ctypes.CDLL(os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "libamdhip64.so"))
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+
+    m = net(6)
+    m.screen_grid(64, 64, tol=0.05, dilate=1)
+    before = free()
+    m.screen_grid(3000, 2900, tol=0.05, dilate=1)  # 8.7 M cells, 122 MB of outputs
+    assert before - free() < 32 << 20
 
 
 @pytest.mark.parametrize("heads", ["all classes tie", "ties across the halves", "far apart", "infinite"])
