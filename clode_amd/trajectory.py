@@ -11,7 +11,7 @@ from typing import Any, Callable, Dict, List, Optional, Tuple, Union
 import numpy as np
 from numpy.lib import recfunctions as rfn
 
-from .cpp.clode_cpp_wrapper import SolverParams, TrajectorySimulatorBase
+from .cpp.clode_cpp_wrapper import SolverParams, TrajectorySimulatorBase, member_rows
 from .runtime import CLDeviceType, CLVendor, _clode_root_dir
 from .solver import Simulator, Stepper
 
@@ -118,22 +118,22 @@ class TrajectorySimulator(Simulator):
         store = self._sp.max_store
         n = self._ensemble_size
         # every member's samples are rows of one array per kind, transposed to
-        # that order on the device; the members' outputs are slices of them
+        # that order on the device; each output has a copy of its own rows
         t = self._integrator.get_t_members()
         if t.shape[1] < store:
             raise ValueError(f"{t.shape[1]} samples per member are stored, max_store is {store}")
-        t = t[:, :store]
         x, dx, aux = (get() for get in (self._integrator.get_x_members, self._integrator.get_dx_members,
                                         self._integrator.get_aux_members))
-        self._device_t = t
+        self._device_t = t[:, :store]
         self._device_x, self._device_dx, self._device_aux = (a.transpose(0, 2, 1)[:, :, :store] for a in (x, dx, aux))
         names, aux_names = self.variable_names, self.aux_names
-        xs, dxs = (a.view(_struct(names))[..., 0] for a in (x, dx))
-        auxs = aux.view(_struct(aux_names))[..., 0] if len(aux_names) > 0 else None
+        counts = np.minimum(np.array(self._integrator.get_n_stored()) + 1, store).tolist()
         make = TrajectoryOutput._of_structured
-        results = []
-        n_stored = np.array(self._integrator.get_n_stored())
-        for i, k in enumerate(np.minimum(n_stored + 1, store).tolist()):
-            results.append(make(t[i, :k], xs[i, :k], dxs[i, :k], auxs[i, :k] if auxs is not None else None, names,
-                                aux_names))
-        return results[0] if n == 1 else results
+        if n == 1:  # its rows are the arrays' first
+            k = counts[0]
+            return make(t[0, :k], x.view(_struct(names))[0, :k, 0], dx.view(_struct(names))[0, :k, 0],
+                        aux.view(_struct(aux_names))[0, :k, 0] if len(aux_names) > 0 else None, names, aux_names)
+        ts = member_rows(t, counts, np.dtype(np.float64))
+        xs, dxs = (member_rows(a, counts, _struct(names)) for a in (x, dx))
+        auxs = member_rows(aux, counts, _struct(aux_names)) if len(aux_names) > 0 else [None] * n
+        return [make(*member, names, aux_names) for member in zip(ts, xs, dxs, auxs)]

@@ -14,6 +14,41 @@ from clode_amd.cpp import clode_cpp_wrapper as w
 MODELS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "clode_amd", "models")
 
 
+def test_member_rows():
+    """Each member's first rows as an array of its own, with the type of a row."""
+    a = np.random.default_rng(0).random((4, 5, 2))
+    dt = np.dtype({"names": ["u", "v"], "formats": [np.float64] * 2})
+    rows = w.member_rows(a, [5, 0, 3, 1], dt)
+    assert [r.shape for r in rows] == [(5,), (0,), (3,), (1,)] and all(r.dtype == dt for r in rows)
+    for i, r in enumerate(rows):
+        assert np.array_equal(r["u"], a[i, :len(r), 0]) and np.array_equal(r["v"], a[i, :len(r), 1])
+        assert r.flags.owndata and r.flags.writeable and not np.shares_memory(r, a)
+    flat = w.member_rows(a[:, :, 0].copy(), [1, 2, 3, 4], np.dtype(np.float64))
+    assert [r.tolist() for r in flat] == [a[i, :i + 1, 0].tolist() for i in range(4)]
+    for bad in (([6, 0, 0, 0], dt), ([-1, 0, 0, 0], dt), ([1, 1, 1], dt), ([1, 1, 1, 1], np.dtype(np.float64))):
+        with pytest.raises(ValueError):
+            w.member_rows(a, *bad)
+
+
+@pytest.mark.gpu
+def test_outputs_own_their_samples(gpu_available):
+    """An output of an ensemble keeps its own samples alone: writing into one changes neither the others nor what the
+    simulator holds."""
+    sim = clode.TrajectorySimulator(src_file=os.path.join(MODELS, "van_der_pol.cl"), variables={"x": 1.0, "y": 0.0},
+                                    parameters={"mu": 1.0}, dt=0.01, stepper=clode.Stepper.rk4, t_span=(0.0, 0.2),
+                                    max_store=50, single_precision=False)
+    sim.set_ensemble(variables={"x": np.linspace(0.5, 2.0, 5)})
+    out = sim.trajectory()
+    held = {k: getattr(sim, "_device_" + k).copy() for k in ("t", "x", "dx")}
+    other = out[3].to_ndarray("x").copy()
+    for slot in ("t", "x", "dx"):
+        a = getattr(out[2], slot)
+        assert a.base is None and len(a) < 50
+        a[:] = 0
+    assert all(np.array_equal(getattr(sim, "_device_" + k), held[k], equal_nan=True) for k in held)
+    assert np.array_equal(out[3].to_ndarray("x"), other)
+
+
 def test_getters_before_any_data():
     """Empty results before problem data are set, also where there is no device."""
     pi = w.ProblemInfo(os.path.join(MODELS, "van_der_pol.cl"), ["x", "y"], ["mu"], [], 0)
