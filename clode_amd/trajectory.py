@@ -49,7 +49,7 @@ class TrajectoryOutput:
 
     def to_ndarray(self, slot: str, **kwargs) -> np.ndarray:
         a = getattr(self, slot)
-        if not kwargs and a.flags.c_contiguous and a.dtype.names is not None:
+        if not kwargs and a.flags.c_contiguous and a.dtype.names is not None and a.dtype == _struct(a.dtype.names):
             # fields of double, one after the other: the same memory as columns
             return a.view(np.float64).reshape(a.shape + (len(a.dtype.names),))
         return rfn.structured_to_unstructured(a, **kwargs)

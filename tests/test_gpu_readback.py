@@ -181,3 +181,14 @@ def test_two_threads_read_one_simulator(gpu_available):
     for t in threads:
         t.join()
     assert wrong == []
+
+
+def test_to_ndarray_of_replaced_samples():
+    """A slot that was given an array of other field types is converted, not reinterpreted."""
+    x = np.arange(10.0).reshape(5, 2)
+    out = clode.TrajectoryOutput(t=np.arange(5.0), x=x, dx=-x, aux=np.empty((5, 0)), variable_names=["u", "v"], aux_names=[])
+    assert np.array_equal(out.to_ndarray("x"), x) and out.to_ndarray("x").dtype == np.float64
+    out.x = out.x.astype([("u", np.float32), ("v", np.float32)])
+    assert np.array_equal(out.to_ndarray("x"), x)
+    out.dx = out.dx.astype([("u", np.int64), ("v", np.float64)])
+    assert np.array_equal(out.to_ndarray("dx"), -x)
