@@ -33,6 +33,7 @@
 
 #include "../../../include/clode_mlp.h"
 #include "../runtime/staged_copy.h"
+#include "normals.h"
 
 // Staging memory of clode_mlp_screen_grid_noalloc: one byte per grid cell for
 // the dilation's second flag buffer.  Each device holds its own copy of the
@@ -1660,45 +1661,6 @@ float loss_grad(clode_mlp *h, int n)
     return l;
 }
 
-// Standard normal deviates by the polar method (Marsaglia and Bray 1964), two
-// from each accepted point of the unit disc, the second coordinate's first.  The
-// values are those that std::normal_distribution<float> gives here; that one
-// works out the generator's range in long double for every draw, 30 ns of them,
-// and a network's 230,000 initial weights took 7 of the 9 ms of its creation.
-class Normals {
-    std::mt19937_64 rng;
-    float kept = 0.f;
-    bool have = false;
-    float uniform()  // [0, 1)
-    {
-        // through a signed conversion, the lost bit kept as a sticky one: the
-        // unsigned conversion branches on a random bit
-        const uint64_t w = rng();
-        const float u = w >> 32 ? (float)(int64_t)(w >> 1 | (w & 1)) * 0x1p-63f : (float)(int64_t)w * 0x1p-64f;
-        return u < 1.f ? u : 0x1.fffffep-1f;
-    }
-
-public:
-    explicit Normals(unsigned long long seed) : rng(seed) {}
-    float operator()()
-    {
-        if (have) {
-            have = false;
-            return kept;
-        }
-        float x, y, r2;
-        do {
-            x = 2.f * uniform() - 1.f;
-            y = 2.f * uniform() - 1.f;
-            r2 = x * x + y * y;
-        } while (r2 > 1.f || r2 == 0.f);
-        const float scale = std::sqrt(-2.f * std::log(r2) / r2);
-        kept = x * scale;
-        have = true;
-        return y * scale;
-    }
-};
-
 // a caller's pointer that must not be null
 template <class T>
 T *need(T *p, const char *what)
@@ -1835,7 +1797,7 @@ int clode_mlp_create(clode_mlp **out, int device, unsigned long long seed)
         }
         h->nparam = off;
         // He-style initialisation for SiLU layers, small heads; Fourier frequencies ~ N(0, 3^2)
-        Normals nd01(seed);
+        clode::Normals nd01(seed);
         std::vector<float> p(h->nparam, 0.f);
         std::vector<uint8_t> mask(h->nparam, 1);
         for (int l = 0; l < NLAYER; ++l) {

@@ -2,6 +2,7 @@
 replace still compiles, and that the quotients by constants are those of IEEE division."""
 import os
 import subprocess
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -186,18 +187,29 @@ def test_quotients_by_constants(tmp_path, divisor, precision):
         near = (m * c).astype(T)
         near = (near.view(U) + r.integers(0, 5, near.size).astype(U) - U(2)).view(T)
         special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, tiny, -tiny, big, -big, 1.0, c, -c, c * tiny], T)
-        p = np.concatenate([anybits, near, special])
+        # subnormal numerators and quotients: small multiples of the smallest one, and of it times half the divisor
+        unit = np.nextafter(T(0), T(1))
+        small = np.arange(-2000, 2001).astype(T) * unit
+        edge = ((2 * np.arange(1000) + 1) * (np.abs(c) / T(2))).astype(T) * unit
+        p = np.concatenate([anybits, near, special, small, edge])
         want = p / c
         got = _quotients(tmp_path, divisor, p, precision).astype(T)
-    # a subnormal quotient by an even number may be a middle itself: either neighbour is as near
-    tie = np.zeros(p.size, bool)
-    if c != 0 and float(c) % 2 == 0 and abs(float(c)) > 2:
-        tie = (np.abs(want) < tiny) & np.isfinite(want)
-        unit = np.nextafter(T(0), T(1))
-        assert np.all(np.abs(got[tie] - want[tie]) <= unit)
+    # by a whole constant the quotient is formed by multiplication; where the true one is the middle between two
+    # subnormals (found in whole numbers of the smallest one), it goes to the neighbour nearer to zero instead of the
+    # even one.  Every other quotient is IEEE's, bit for bit
+    middle = np.zeros(p.size, bool)
+    y = abs(int(c)) if c == np.trunc(c) else 0
+    if y and y < (2 ** 19 if precision else 2 ** 48) and y & (y - 1):
+        unit = float(np.nextafter(T(0), T(1)))
+        for i in np.flatnonzero(np.isfinite(p) & (np.abs(want) <= tiny)):
+            x = int(abs(Fraction(float(p[i])) / Fraction(unit)))
+            if 2 * x % y == 0 and 2 * x // y % 2:
+                middle[i] = True
+                want[i] = np.copysign(T(x // y * unit), want[i])
+        assert middle.any() == (y % 2 == 0)
     want = want + T(0)  # x = 0 + 1 * (p / c)
     same = (got.view(U) == want.view(U)) | (np.isnan(got) & np.isnan(want))
-    assert np.all(same | tie), (p[~(same | tie)][:5], got[~(same | tie)][:5], want[~(same | tie)][:5])
+    assert np.all(same), (p[~same][:5], got[~same][:5], want[~same][:5], middle[~same][:5])
 
 
 @pytest.mark.gpu
