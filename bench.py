@@ -22,9 +22,11 @@ Extra workloads (--extras, default all): fp32c (the headline in fp32c), seq
 the warm-up's recorded steps from HBM), c1
 (Van der Pol 4096, rk4), noise (the lactotroph Euler-Maruyama variant),
 c3 (Lorenz 2^20, and the 65,536 x 1024-sample trajectory), c4 (mixed 2^20
-batched sweep), c5 (surrogate-screened 2048 x 2048 map).
+batched sweep), c5 (surrogate-screened 2048 x 2048 map).  Their figures go to
+stderr, one line each (and to --extra-json); the JSON line names them.
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-extra] [--extras LIST]
+                       [--extra-json FILE]
 """
 from __future__ import annotations
 
@@ -737,6 +739,15 @@ def profiled_traffic(kernel="clode_features"):
     return int(m.group(1)) if m else None
 
 
+def short(v):
+    """v with every float at six significant digits (but the two that the line is read for)."""
+    if isinstance(v, float):
+        return float(f"{v:.6g}")
+    if isinstance(v, dict):
+        return {k: x if k in ("value", "ms_per_step") else short(x) for k, x in v.items()}
+    return v
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -750,6 +761,7 @@ def main():
                          "replay), c1, noise, c3, c4, c5 "
                          "(or 'none'); --no-extra "
                          "drops them all")
+    ap.add_argument("--extra-json", help="also write the extra workloads' figures to this file")
     ap.add_argument("--c4-rounds", type=int, default=8)
     ap.add_argument("--mlp-kernels", action="store_true",
                     help="run only the surrogate kernels (one training epoch over 65,536 synthetic samples and one "
@@ -834,7 +846,7 @@ def main():
             extra[name] = fn()
         except Exception as e:  # an extra figure must not cost the headline line
             extra[name] = {"error": f"{type(e).__name__}: {e}"}
-        print(f"# {name}: {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
+        print(f"# {name}: {time.perf_counter() - t0:.1f} s {json.dumps(extra[name])}", file=sys.stderr, flush=True)
 
     r32 = None
     if "fp32c" in wanted:
@@ -909,9 +921,14 @@ def main():
         "map_2048": maps or None,
         "roofline": roofline,
         "cpu_baseline": cpu,
-        "extra": extra,
+        "extra": sorted(extra),
+        "extra_errors": sorted(k for k, v in extra.items() if "error" in v) or None,
     }
-    print(json.dumps(line), flush=True)
+    if args.extra_json:
+        with open(args.extra_json, "w") as f:
+            json.dump(extra, f, indent=1)
+    # short enough for a log that keeps the end of the output: six digits, the extra workloads' figures on stderr
+    print(json.dumps(short(line)), flush=True)
 
 
 if __name__ == "__main__":
