@@ -6,6 +6,7 @@ only (clode/trajectory.py:18-266).
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Any, Callable, Dict, List, Optional, Tuple, Union
 
 import numpy as np
@@ -16,8 +17,14 @@ from .runtime import CLDeviceType, CLVendor, _clode_root_dir
 from .solver import Simulator, Stepper
 
 
+@lru_cache(maxsize=256)
+def _fields(names: Tuple[str, ...]) -> np.dtype:
+    return np.dtype({"names": list(names), "formats": [np.float64] * len(names)})
+
+
 def _struct(names: List[str]) -> np.dtype:
-    return np.dtype({"names": names, "formats": [np.float64] * len(names)})
+    """A row of doubles with these names: the same object for the same names, which compares fastest."""
+    return _fields(tuple(names))
 
 
 class TrajectoryOutput:
@@ -49,9 +56,10 @@ class TrajectoryOutput:
 
     def to_ndarray(self, slot: str, **kwargs) -> np.ndarray:
         a = getattr(self, slot)
-        if not kwargs and a.flags.c_contiguous and a.dtype.names is not None and a.dtype == _struct(a.dtype.names):
+        names = a.dtype.names
+        if not kwargs and names is not None and a.dtype == _fields(names) and a.flags.c_contiguous:
             # fields of double, one after the other: the same memory as columns
-            return a.view(np.float64).reshape(a.shape + (len(a.dtype.names),))
+            return a.view(np.float64).reshape(a.shape + (len(names),))
         return rfn.structured_to_unstructured(a, **kwargs)
 
 

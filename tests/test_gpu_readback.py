@@ -15,16 +15,24 @@ MODELS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))
 
 
 def test_member_rows():
-    """Each member's first rows as an array of its own, with the type of a row."""
+    """Each member's first rows as an array with the type of a row, copied, in blocks of at most 64 KiB."""
     a = np.random.default_rng(0).random((4, 5, 2))
     dt = np.dtype({"names": ["u", "v"], "formats": [np.float64] * 2})
     rows = w.member_rows(a, [5, 0, 3, 1], dt)
     assert [r.shape for r in rows] == [(5,), (0,), (3,), (1,)] and all(r.dtype == dt for r in rows)
     for i, r in enumerate(rows):
         assert np.array_equal(r["u"], a[i, :len(r), 0]) and np.array_equal(r["v"], a[i, :len(r), 1])
-        assert r.flags.owndata and r.flags.writeable and not np.shares_memory(r, a)
+        assert r.flags.writeable and r.flags.c_contiguous and not np.shares_memory(r, a)
+    assert not any(np.shares_memory(r, q) for r in rows for q in rows if r is not q and len(r) and len(q))
     flat = w.member_rows(a[:, :, 0].copy(), [1, 2, 3, 4], np.dtype(np.float64))
     assert [r.tolist() for r in flat] == [a[i, :i + 1, 0].tolist() for i in range(4)]
+    many = np.arange(700 * 40.0).reshape(700, 40)
+    counts = [(7 * i) % 41 for i in range(700)]
+    rows = w.member_rows(many, counts, np.dtype(np.float64))
+    assert all(np.array_equal(r, many[i, :counts[i]]) and r.base.nbytes <= 65536 for i, r in enumerate(rows))
+    assert len({id(r.base) for r in rows if r.size}) == -(-sum(counts) * 8 // 65536)
+    large = w.member_rows(np.ones((3, 9000)), [9000, 1, 8999], np.dtype(np.float64))
+    assert [r.size for r in large] == [9000, 1, 8999] and [r.base.size for r in large] == [9000, 1, 8999]
     for bad in (([6, 0, 0, 0], dt), ([-1, 0, 0, 0], dt), ([1, 1, 1], dt), ([1, 1, 1, 1], np.dtype(np.float64))):
         with pytest.raises(ValueError):
             w.member_rows(a, *bad)
@@ -32,7 +40,7 @@ def test_member_rows():
 
 @pytest.mark.gpu
 def test_outputs_own_their_samples(gpu_available):
-    """An output of an ensemble keeps its own samples alone: writing into one changes neither the others nor what the
+    """An output of an ensemble has a copy of its samples, in a block of at most 64 KiB: writing into one changes neither the others nor what the
     simulator holds."""
     sim = clode.TrajectorySimulator(src_file=os.path.join(MODELS, "van_der_pol.cl"), variables={"x": 1.0, "y": 0.0},
                                     parameters={"mu": 1.0}, dt=0.01, stepper=clode.Stepper.rk4, t_span=(0.0, 0.2),
@@ -43,7 +51,7 @@ def test_outputs_own_their_samples(gpu_available):
     other = out[3].to_ndarray("x").copy()
     for slot in ("t", "x", "dx"):
         a = getattr(out[2], slot)
-        assert a.base is None and len(a) < 50
+        assert a.base.nbytes <= 65536 and len(a) < 50
         a[:] = 0
     assert all(np.array_equal(getattr(sim, "_device_" + k), held[k], equal_nan=True) for k in held)
     assert np.array_equal(out[3].to_ndarray("x"), other)
