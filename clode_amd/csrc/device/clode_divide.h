@@ -22,12 +22,13 @@
 // side), 65,536 members, dopri5, double, transient + warm-up + features
 // 180.1 -> 164.0 ms; 1,000 members, rk4, single, 5.98 -> 4.85 ms; van der Pol,
 // 4,096 members, rk4, double (2 in the update), 8.31 -> 7.43 ms.  The same
-// bits everywhere.
+// bits but for those subnormal middles.
 //
 // Right-hand sides are written with "/": the program builder replaces the
 // token by "*CLODE_DIV*" inside function bodies (same precedence, same
-// associativity), and the operators below give every pair of arithmetic types
-// the value of "/".  Which path a division takes is decided by the optimiser:
+// associativity), and the operators below give every pair of types the value
+// of "/": a pair of arithmetic types through divide(), any other through its own
+// operator.  Which path a division takes is decided by the optimiser:
 // a divisor that is not a constant there takes the ordinary division.
 #ifndef CLODE_DIVIDE_H
 #define CLODE_DIVIDE_H

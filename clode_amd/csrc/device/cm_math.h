@@ -85,7 +85,9 @@ CM_FN double exp(double x)
     double xc = clamp_num(x, -746.0, 710.0);
     // k = x log2 e rounded to a whole number by adding 1.5 2^52, which also
     // leaves k in the low bits of the sum (two instructions for the product,
-    // the rounding and the conversion to int)
+    // the rounding and the conversion to int).  One rounding instead of the two
+    // of rint(xc * log2e): for a few x next to (k + 1/2) ln 2 the other k, with
+    // r as close to ln2/2 and a result at most 1 ulp from the other
     const double shift = 0x1.8p52;
     double ks = fma(xc, log2e, shift);
     double k = ks - shift;

@@ -7,10 +7,12 @@
 // their own pinned block (57 GB/s in all) and copy it out, so that the page
 // faults of several chunks are served at once.
 //
-// The pinned blocks (THREADS x CHUNK = 12 MiB) are shared by everything that
-// holds a StagedCopy and freed with its last holder.  One copy uses them at a
-// time; a second one at the same moment, a small copy, or one for which no
-// threads or pinned memory are to be had takes the runtime's copy.  The
+// The pinned blocks (THREADS x CHUNK = 12 MiB) are allocated by the first large
+// copy, shared by everything in a library that holds a StagedCopy and freed
+// with its last holder; the integrator's library and the surrogate's have blocks
+// of their own.  One copy uses a library's blocks at a time; a second one at the
+// same moment, a small copy, or one for which no threads or pinned memory are to
+// be had takes the runtime's copy.  The
 // device work that produces the data must have been queued on `stream` before;
 // the copies are queued there too, and the call returns when all have arrived.
 #pragma once

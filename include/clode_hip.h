@@ -190,8 +190,11 @@ int clode_get_t(clode_sim *sim, double *out, size_t n);
 int clode_get_x(clode_sim *sim, double *out, size_t n);
 int clode_get_dx(clode_sim *sim, double *out, size_t n);
 int clode_get_aux(clode_sim *sim, double *out, size_t n);
-/* the same member by member (transposed on the device): t [nPts][max_store],
- * x and dx [nPts][max_store][num_var], aux [nPts][max_store][num_aux] */
+/* the same member by member (transposed on the device, through a block of at
+ * most 256 MiB, or CLODE_MEMBERS_BYTES from the environment; on the host where
+ * there is no room for a block): t [nPts][max_store], x and dx
+ * [nPts][max_store][num_var], aux [nPts][max_store][num_aux].  Threads that read
+ * one simulator this way at the same time wait for each other. */
 int clode_get_t_members(clode_sim *sim, double *out, size_t n);
 int clode_get_x_members(clode_sim *sim, double *out, size_t n);
 int clode_get_dx_members(clode_sim *sim, double *out, size_t n);

@@ -63,7 +63,9 @@ int clode_mlp_train(clode_mlp *h, const float *X, const float *T, const int *cls
 /* Screen the nx x ny grid of normalised inputs (ix / (nx - 1), iy / (ny - 1)),
  * cell index ix * ny + iy: ensemble period, amplitude and class per cell, and
  * flags (bit 0 heads disagree by more than tol, bit 1 class differs from a
- * 4-neighbour, bit 2 within `dilate` cells of a flagged cell) */
+ * 4-neighbour, bit 2 within `dilate` cells of a flagged cell).  Up to 2^23
+ * cells the device buffers stay with the network (14 bytes per cell).  Threads
+ * that screen with one network at the same time wait for each other. */
 int clode_mlp_screen_grid(clode_mlp *h, int nx, int ny, float tol, int dilate, float *period, float *amp, int *cls,
                           unsigned char *flags);
 /* device time of the last train / screen call, milliseconds */
